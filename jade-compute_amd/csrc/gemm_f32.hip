@@ -2426,10 +2426,9 @@ hipError_t gemm_f32_dual_swiglu(hipStream_t stream, const float *a, const float 
     const int edge_n = dual_edge_columns(tiles_m, tiles_n), body_tn = tiles_n - edge_n;
     const unsigned grid = unsigned(tiles_m * body_tn + 2 * tiles_m * edge_n);
     if (route_for(m, n, k).plan.ring)
-        hipLaunchKernelGGL(gemm_f32_dual_swiglu<ring::kFoldRun>, dim3(grid), dim3(dual::kThreads), 0, stream, a, bg,
-                           bu, g, u, act, int(n), int(k), tiles_m, tiles_n, body_tn);
-    else
-        hipLaunchKernelGGL(gemm_f32_dual_swiglu<kFoldStages>, dim3(grid), dim3(dual::kThreads), 0, stream, a, bg,
+        return launch_gemm_ring_swiglu(stream, a, bg, bu, g, u, act, n, k, tiles_m, tiles_n,
+                                       unsigned(std::min(tiles_m * tiles_n, kCUs)));
+    hipLaunchKernelGGL(gemm_f32_dual_swiglu<kFoldStages>, dim3(grid), dim3(dual::kThreads), 0, stream, a, bg,
                            bu, g, u, act, int(n), int(k), tiles_m, tiles_n, body_tn);
     return hipGetLastError();
 }

@@ -1,96 +1,74 @@
 // FP32 GEMM on persistent 128x128 tiles for large products whose grid
 // covers every CU: C[M,N] = A[M,K] * B[K,N], packed row-major, the same
-// contract as gemm_f32.hip (src/runtime/ir.rs:21-32). Built as its own
-// translation unit so that its MFMAs accumulate in architectural VGPRs
-// (-mllvm -amdgpu-mfma-vgpr-form=1 in the Makefile): the fold of a run into
-// the running sums then reads the accumulators directly instead of through
-// v_accvgpr_read.
+// contract as gemm_f32.hip (src/runtime/ir.rs:21-32).
 #include <type_traits>
 
 #include "gemm_tiles.hpp"
+#include "ops.hpp"
+#include "split_bf16.hpp"
 
 namespace jade {
 namespace hipk {
 namespace {
 
-// ---- Persistent 128x128 tiles: one workgroup per CU, a four-stage LDS ring ----
+// ---- Persistent 128x128 tiles: one workgroup per CU, products on bf16 parts ----
+// What bounds it: the bf16 matrix cores (six v_mfma_f32_32x32x16_bf16 per
+// FP32 product block, split_bf16.hpp), at 1.8-2.0 GHz: a chip full of them
+// runs 1.81 PFLOP/s with one wave per SIMD and 1.98 with two, so 300-330
+// TFLOP/s of FP32 products. v_mfma_f32_32x32x2_f32, which this kernel ran on
+// before, tops out at 157 and this kernel reached 150 with it.
+// Measured (us, one box, against that kernel): 4096^3 918 -> 684, 2048^3
+// 120.0 -> 91, 4096x11008x4096 2490 -> 1880. With the staging taken out of a
+// copy (MFMAs and operand reads alone) 4096^3 runs 437 us; global loads, the
+// conversion and the LDS writes each add 60-90 us of issue and waiting that
+// the two waves of a SIMD do not hide. Neither the order of that work (spread
+// one piece per MFMA as here 672, all before the MFMAs 701, after 730, left to
+// the compiler 706) nor a third stage buffer with the writes a whole stage
+// ahead of their barrier (735) changes it much; four waves of 64x64 (one per
+// SIMD) ran 716, and 256x128 tiles spill.
+//
 // A launch of at most one workgroup per CU; workgroup b takes the tiles
 // pos(b), pos(b) + G, pos(b) + 2G, ... of the XCD-grouped order (G workgroups,
 // pos the XCD-contiguous position), so each XCD's 32 workgroups work on a
-// block of 8 tile rows x 4 tile columns at a time. The workgroup's stages form
-// one sequence over all its tiles; stage g+3 is loaded (LDS-direct) into the
-// ring while stage g is consumed, so loads run across tile boundaries and the
-// epilogue of one tile overlaps the first stage of the next.
+// block of 8 tile rows x 4 tile columns at a time. The workgroup's 32-k stages
+// form one sequence over all its tiles: loads and conversions run ahead
+// across tile boundaries.
 //
-// Eight waves of 32x64 (two blocks of v_mfma_f32_32x32x2_f32 each, two waves
-// per SIMD), 128 KiB of LDS: four 32-deep stages (A regions in the first 64
-// KiB, B regions in the second). Per stage:
-//  * one barrier, after this wave's loads of stage g+1 have landed: it
-//    publishes stage g+1 and retires stage g-1's slot, which stage g+3's loads
-//    fill while stage g is consumed, one load after every eight MFMAs;
-//  * the operands of quarter q+1 (8 k) are read one after each of quarter q's
-//    first MFMAs, and quarter 0 of stage g+1 during quarter 3 of stage g, so
-//    no MFMA waits on an LDS read after the barrier;
-//  * every LDS operand address is a per-lane constant plus an immediate (12
-//    address registers), and the load offsets are per-lane constants plus a
-//    uniform base, so the loop carries no VALU address arithmetic;
-//  * no branch: every stage issues its loads (past the end of the sequence
-//    they re-read the last tile into a slot nothing reads), the load cursor
-//    advances by selects, and each tile's first iteration, which stores the
-//    previous tile, is a separate instantiation of the eight-stage body.
-// Accumulation is the LDS-direct loops' two-level scheme with their MFMA
-// order and a longer run: runs of kFoldRun (eight) stages sum in MFMA
-// accumulators and are folded into the running sums with VALU adds, where the
-// tile loops fold every four stages. The fold of a block sits right before
-// that block's first MFMA of the next run. The fused gate/up kernel takes the
-// same run length where it stands in for this kernel, so its outputs stay
-// bit-identical to this kernel's.
+// Eight waves of 32x64 (two 32x32 blocks each, two waves per SIMD). Each
+// element of a stage is loaded and split once per workgroup: FP32 from global
+// memory into registers two stages ahead, three bf16 parts into LDS (48 KiB a
+// stage, two stages). A row (and B column) of a part is 64 bytes of LDS, k
+// contiguous, its four 16-byte chunks XORed with (row >> 2) & 3, so that an
+// operand read (16 rows at one chunk) covers all banks. B column 64w + 2c + j
+// of the tile is LDS row 64w + 32j + c: a lane's outputs of blocks 0 and 1 are
+// then adjacent columns, and the lanes that write B write adjacent rows.
 //
-// Measured at 4096^3 (TFLOP/s, A/B on one box; the non-persistent 128x128
-// kernel ran 141.6): first form, four waves of 64x64 with all of a stage's
-// loads at its top, 133.1; loads spread one per eight MFMAs, 136.9; no branch
-// in the steady state (the first form carried ~12 branches and ~84 scalar
-// instructions per stage), 145.7; operand reads interleaved with the MFMAs
-// instead of issued back to back (the waves then waited on the LDS pipe four
-// times as long as the library's kernel), 147.4 with four waves and 149.3 with
-// eight; runs of eight stages instead of four before each fold (kFoldRun),
-// 149.4; each load after the seventh of its eight MFMAs instead of the last,
-// 150.5 (identical bits; 4096x11008x4096 -0.7% time, 2048^3 -0.5%).
-// Halving the barriers (a timing-only copy without the odd stages' barriers)
-// and folding the two waves of a SIMD at different stages (so one
-// wave's MFMAs cover the other's fold) were measured and changed nothing.
-// Also measured and dropped: raised wave priority over each stage's matrix
-// work (s_setprio; 4096^3 913.95 -> 915.15 us, 4096x11008x4096 -0.4%);
-// sixteen waves of 32x32 (four per SIMD), 1%
-// slower at every shape; 128x256 tiles of 16-deep stages (eight waves of
-// 32x128: half the operand reads per MFMA), 4096^3 918.5 -> 929 us.
-// Requires M, N multiples of 128, K a multiple of 256 (whole eight-stage
-// iterations per tile), 16-byte aligned operands, 32-bit load offsets.
+// Accumulation is two-level: runs of kFoldRun stages (256 k) sum in the MFMA
+// accumulators, small products first, and are folded into the running sums
+// with VALU adds. Error against FP64 (2-norm, relative, uniform [-1, 1)):
+// 4096^3 2.5e-7 (the FP32 MFMAs 3.0e-7), 2048^3 2.4e-7 (3.0e-7).
+//
+// Values the parts do not carry: below 2^-100 the third part meets bf16's
+// smallest subnormal, an infinity minus its own first part is NaN, and at the
+// top of the range the partial products overflow one by one. So every tile
+// that read a nonzero value below 2^-100, and every wave whose sums are not
+// all finite, computes its outputs again from global memory with FP32 MFMAs:
+// infinities, NaN, overflow and tiny operands come out as FP32 arithmetic
+// gives them, at about a tenth of the speed.
+//
+// Requires M, N multiples of 128 (N of 64 for DUAL), K a multiple of 256,
+// 16-byte aligned operands, 32-bit load offsets inside a tile.
 namespace ring_local {
 using namespace ring;
-static_assert(kUnroll % kFoldRun == 0 && kUnroll % kDepth == 0, "slot and run start are compile-time per stage");
+using namespace split;
 
-// One quarter of a stage's operands for one lane: a[i] = A[row block i][k
-// 16h + 4q + e] at a[i][e]; b[e] = B[k 16h + 4q + e][columns 2c, 2c + 1].
-template <int TM>
-struct Quarter {
-    f32x4 a[TM];
-    float2 b[4];
+// One half-stage's operands (16 k) for one lane: part p of the A row block and
+// of B column block j, eight consecutive k each.
+struct Operands {
+    bf16x8 a[kParts], b[2][kParts];
 };
 
-// s_waitcnt vmcnt(N), then the workgroup barrier.
-template <int N>
-__device__ inline void wait_loads_barrier() {
-    static_assert(N == 0 || N == 4 || N == 8 || N == 16, "wait counts in use");
-    if constexpr (N == 0)
-        asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-    else if constexpr (N == 4)
-        asm volatile("s_waitcnt vmcnt(4)\n\ts_barrier" ::: "memory");
-    else if constexpr (N == 8)
-        asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");
-    else
-        asm volatile("s_waitcnt vmcnt(16)\n\ts_barrier" ::: "memory");
-}
+constexpr uint32_t kRawBuffer = 0x00020000;  // buffer descriptor word 3: raw buffer, 32-bit data format
 
 __device__ inline int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 __device__ inline const float *uniform(const float *p) {
@@ -98,292 +76,379 @@ __device__ inline const float *uniform(const float *p) {
     const uint32_t lo = __builtin_amdgcn_readfirstlane(uint32_t(v)), hi = __builtin_amdgcn_readfirstlane(uint32_t(v >> 32));
     return reinterpret_cast<const float *>((uint64_t(hi) << 32) | lo);
 }
+// Position of logical 16-byte chunk j (eight k) in a 64-byte LDS row.
+__device__ inline int swz(int row) { return (row >> 2) & 3; }
 }  // namespace ring_local
 
-// TM: MFMA row blocks per wave. A wave computes (32 TM) x 64 of the tile; the
-// workgroup has 8 / TM waves as (4 / TM) x 2 (TM = 2: four waves of 64x64,
-// one per SIMD; TM = 1: eight waves of 32x64, two per SIMD).
-// PAIRS: C is 8-byte aligned, so each lane's two adjacent outputs go out as
-// one 8-byte store.
-// sum != nullptr: the epilogue also stores sum = C + residual (both [M, N]),
-// the stream kernel's FP32 add, so `sum` is bit-identical to an Add launched
-// after the product.
-template <int TM, bool PAIRS>
-__global__ __launch_bounds__(512 / TM) __attribute__((amdgpu_waves_per_eu(3 - TM, 3 - TM))) void gemm_f32_ring(
-    const float *__restrict__ A, const float *__restrict__ B, float *__restrict__ C, int N, int K, int tiles_m,
-    int tiles_n, const float *__restrict__ residual, float *__restrict__ sum) {
+// Plain stores single floats; Pairs stores each lane's two adjacent outputs as
+// 8 bytes (C, residual and sum 8-byte aligned). Both store sum = C + residual
+// as well where sum is not null (the stream kernel's FP32 add, so `sum` is
+// bit-identical to an Add launched after the product). Dual computes 128x64
+// tiles of two products of one A (B into C, B2 into C2), the operand columns
+// of both side by side, and their SwiGLU into sum; every output takes the
+// steps over k that its product takes alone.
+enum class RingForm { Plain, Pairs, Dual };
+
+template <RingForm FORM>
+__global__ __launch_bounds__(ring::kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_f32_ring(
+    const float *__restrict__ A, const float *__restrict__ B, const float *__restrict__ B2, float *__restrict__ C,
+    float *__restrict__ C2, int N, int K, int tiles_m, int tiles_n, const float *__restrict__ residual,
+    float *__restrict__ sum) {
     using namespace ring;
     using namespace ring_local;
-    constexpr int kWaves = 8 / TM;
-    constexpr int kLoads = 32 / kWaves;      // one-KiB loads per wave per stage (half A, half B)
-    constexpr int kMfmas = 4 * TM * 2;       // MFMAs per wave per quarter
-    static_assert(kMfmas % 8 == 0 && kLoads == 4 * (kMfmas / 8), "one load per eight MFMAs");
-    __shared__ __attribute__((aligned(1024))) char lds[kLdsBytes];
-    const int lane = int(threadIdx.x) & 63;
-    const int wave = uniform(int(threadIdx.x) >> 6);
+    constexpr bool DUAL = FORM == RingForm::Dual;
+    __shared__ __attribute__((aligned(1024))) char lds[kStages];
+    __shared__ int tiny;  // whether the tile read a value its parts do not carry
+    const int tid = int(threadIdx.x), lane = tid & 63;
+    const int wave = uniform(tid >> 6);
     const int h = lane >> 5, c = lane & 31, wm = wave >> 1, wn = wave & 1;
     const int nwg = int(gridDim.x), tiles = tiles_m * tiles_n;
     const int pos = xcd_order(int(blockIdx.x), nwg);
     const int mine = (tiles - pos + nwg - 1) / nwg;  // tiles pos, pos + nwg, ...
     const int nk = K / kBK;
-    const uint32_t lds0 = lds_address(lds);
+    constexpr int kTileN = DUAL ? kBN / 2 : kBN;
 
-    // Load offsets. A: 16 one-KiB loads of eight 128-byte rows per stage; B:
-    // 16 loads of two 512-byte rows; kLoads / 2 of each per wave. The chunk
-    // swizzles are the LDS-direct tiles' (swz_a, swz_b).
-    constexpr int kHalf = kLoads / 2;
-    uint32_t voa[kHalf], vob[kHalf];
+    // Staging, per thread: one A chunk (row tid / 4, k 8 (tid % 4) on) and
+    // four k (4 wave on) of two B columns.
+    const int ar = tid >> 2, aq = tid & 3;
+    const uint32_t va = uint32_t((ar * K + 8 * aq) * 4);
+    const uint32_t vb = uint32_t((4 * wave * N + (DUAL ? lane : 2 * lane)) * 4), vbk = uint32_t(N) * 4u;
+    const uint32_t wa = uint32_t(ar * 64 + ((aq ^ swz(ar)) << 4));
+    const int br = (lane >> 5) * 64 + c;  // LDS row of the first column; the second is 32 rows on
+    const uint32_t wb = uint32_t(kBRegion + br * 64 + (((wave >> 1) ^ swz(br)) << 4) + (wave & 1) * 8);
+    // Operand reads: A row 32 wm + c, B row 64 wn + 32 j + c, chunk 2 half + h.
+    uint32_t ra[2], rb[2];
 #pragma unroll
-    for (int i = 0; i < kHalf; ++i) {
-        const int inst = wave * kHalf + i;
-        const int ra = inst * 8 + (lane >> 3), ja = (lane & 7) ^ swz_a(ra);
-        voa[i] = uint32_t((ra * K + 4 * ja) * 4);
-        const int rb = inst * 2 + (lane >> 5), jb = (lane & 31) ^ swz_b(rb);
-        vob[i] = uint32_t((rb * N + 4 * jb) * 4);
+    for (int s = 0; s < 2; ++s) {
+        ra[s] = uint32_t((32 * wm + c) * 64 + (((2 * s + h) ^ swz(c)) << 4));
+        rb[s] = uint32_t(kBRegion + (64 * wn + c) * 64 + (((2 * s + h) ^ swz(c)) << 4));
     }
-    // Operand addresses. A row 32 (TM wm + i) + c has swizzle ((c >> 1) & 7)
-    // for every block, so block i is +4 KiB; quarter q reads logical chunk
-    // 4h + q. B row 16h + 4q + e has swizzle 4(q & 1) + e; q >= 2 is +4 KiB.
-    uint32_t aoff[4], boff[2][4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-        aoff[q] = uint32_t((wm * 32 * TM + c) * 128 + (((4 * h + q) ^ ((c >> 1) & 7)) << 4));
-#pragma unroll
-    for (int p = 0; p < 2; ++p)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            boff[p][e] = kBRegion + uint32_t((16 * h + 4 * p + e) * 512 + (((wn * 16 + (c >> 1)) ^ (4 * p + e)) << 4) +
-                                             (c & 1) * 8);
-    // This lane's first output (row 4h of the wave's rows, column 2c of its
-    // columns) relative to a tile's origin; other outputs are rows apart.
-    const uint32_t out_lane = uint32_t((wm * 32 * TM + 4 * h) * N + wn * 64 + 2 * c);
 
-    // Block-uniform load cursor: stage dks of the tile whose A rows start at
-    // da and B columns at db; nda, ndb are the next tile's (the current
-    // one's on the last tile, so that loads issued past the sequence's end,
-    // which nothing reads, stay inside A and B).
-    int dks = 0;
-    const float *da, *db, *nda, *ndb;
     auto tile_origin = [&](int j, int &m0, int &n0) {
         int tm, tn;
-        grouped_tile(j * nwg + pos, tiles_m, tiles_n, tm, tn);
+        grouped_tile(min(j, mine - 1) * nwg + pos, tiles_m, tiles_n, tm, tn);
         m0 = uniform(tm * kBM);
-        n0 = uniform(tn * kBN);
+        n0 = uniform(tn * kTileN);
     };
-    auto bases = [&](int j, const float *&pa, const float *&pb) {
+    // Load cursors: the stage of the next A and of the next B load. Each
+    // wraps to the next tile; past the last tile they run over it again, in
+    // bounds, and those stages are never multiplied.
+    int sa = 0, sb = 0;
+    const float *pa, *pb, *pb2 = nullptr, *next_a, *next_b, *next_b2 = nullptr;
+    {
         int m0, n0;
-        tile_origin(j, m0, n0);
+        tile_origin(0, m0, n0);
         pa = uniform(A + size_t(m0) * size_t(K));
         pb = uniform(B + n0);
+        if (DUAL) pb2 = uniform(B2 + n0);
+    }
+    auto aim_next = [&](int tile) {
+        int m0, n0;
+        tile_origin(tile, m0, n0);
+        next_a = uniform(A + size_t(m0) * size_t(K));
+        next_b = uniform(B + n0);
+        if (DUAL) next_b2 = uniform(B2 + n0);
     };
-    // Load x (A loads first, then B) of the stage at the cursor, into
-    // `slot`; the last one advances the cursor, without a branch. A stage's
-    // loads are spread one per eight MFMAs through the stage that consumes
-    // stage g: a wave that issued them all at once stalled on the memory pipe
-    // while its matrix pipe ran dry.
-    auto issue_part = [&](int slot, int x) {
-        if (x < kHalf) {
-            lds_dma16(da + dks * kBK, voa[x], lds0 + slot * kAStageB + uint32_t((wave * kHalf + x) * 1024));
-        } else {
-            lds_dma16(db + size_t(dks) * kBK * size_t(N), vob[x - kHalf],
-                      lds0 + kBRegion + slot * kBStageB + uint32_t((wave * kHalf + x - kHalf) * 1024));
-            if (x == kLoads - 1) {
-                const bool wrap = dks + 1 == nk;
-                dks = wrap ? 0 : dks + 1;
-                da = wrap ? nda : da;
-                db = wrap ? ndb : db;
-            }
+    aim_next(1);
+    auto buffer = [](const float *base) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(base), 0, -1, int(kRawBuffer));
+    };
+    f32x4 rawa[2][2];
+    f32x2 rawb[2][4];
+    auto load_a = [&](int set, int x) {  // the chunk's float4 x; the last one advances the cursor
+        rawa[set][x] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(buffer(pa), int(va), 16 * x, 0));
+        if (x == 1) {
+            const bool wrap = ++sa == nk;
+            pa = wrap ? next_a : pa + kBK;
+            sa = wrap ? 0 : sa;
         }
     };
-    auto issue_next = [&](int slot) {
-#pragma unroll
-        for (int x = 0; x < kLoads; ++x) issue_part(slot, x);
+    auto load_b = [&](int set, int e) {  // k row e of the thread's four
+        if constexpr (DUAL) {
+            rawb[set][e].x = __builtin_bit_cast(
+                float, __builtin_amdgcn_raw_buffer_load_b32(buffer(pb), int(vb), int(uint32_t(e) * vbk), 0));
+            rawb[set][e].y = __builtin_bit_cast(
+                float, __builtin_amdgcn_raw_buffer_load_b32(buffer(pb2), int(vb), int(uint32_t(e) * vbk), 0));
+        } else {
+            rawb[set][e] = __builtin_bit_cast(
+                f32x2, __builtin_amdgcn_raw_buffer_load_b64(buffer(pb), int(vb), int(uint32_t(e) * vbk), 0));
+        }
+        if (e == 3) {
+            const bool wrap = ++sb == nk;
+            const size_t step = size_t(kBK) * size_t(N);
+            pb = wrap ? next_b : pb + step;
+            if (DUAL) pb2 = wrap ? next_b2 : pb2 + step;
+            sb = wrap ? 0 : sb;
+        }
     };
-    // Read r of a quarter's TM + 4 operand reads (A blocks, then B rows).
-    auto read_part = [&](int slot, int q, int r, Quarter<TM> &o) {
-        if (r < TM)
-            o.a[r] = *reinterpret_cast<const f32x4 *>(lds + aoff[q] + r * 4096 + slot * kAStageB);
-        else
-            o.b[r - TM] =
-                *reinterpret_cast<const float2 *>(lds + boff[q & 1][r - TM] + (q >> 1) * 4096 + slot * kBStageB);
+    // Conversion of pair u of the A chunk (k 2u, 2u + 1) or of B (column
+    // u / 2, k 2 (u % 2) on), in three pieces.
+    uint32_t parts[2][kParts][4];
+    f32x2 rest;
+    u16x2 smallest = {0xffff, 0xffff};
+    auto convert = [&](int is_b, int set, int u, int piece) {
+        if (piece == 0) {
+            f32x2 x;
+            if (is_b) {
+                const f32x2 k0 = rawb[set][2 * (u & 1)], k1 = rawb[set][2 * (u & 1) + 1];
+                x = u < 2 ? f32x2{k0.x, k1.x} : f32x2{k0.y, k1.y};
+            } else {
+                x = f32x2{rawa[set][u >> 1][2 * (u & 1)], rawa[set][u >> 1][2 * (u & 1) + 1]};
+            }
+            const uint32_t p = pack(x.x, x.y);
+            parts[is_b][0][u] = p;
+            rest = f32x2{x.x - low_part(p), x.y - high_part(p)};
+        } else if (piece == 1) {
+            const uint32_t p = pack(rest.x, rest.y);
+            parts[is_b][1][u] = p;
+            rest = f32x2{rest.x - low_part(p), rest.y - high_part(p)};
+        } else {
+            parts[is_b][2][u] = pack(rest.x, rest.y);
+            smallest = __builtin_elementwise_min(smallest, doubled_less_one(parts[is_b][0][u]));
+        }
     };
-    auto read_quarter = [&](int slot, int q, Quarter<TM> &o) {
-#pragma unroll
-        for (int r = 0; r < TM + 4; ++r) read_part(slot, q, r, o);
+    auto write_a = [&](int p, int buf) {
+        *reinterpret_cast<u32x4 *>(lds + wa + uint32_t(p) * kPart + uint32_t(buf) * kStageB) =
+            u32x4{parts[0][p][0], parts[0][p][1], parts[0][p][2], parts[0][p][3]};
     };
+    auto write_b = [&](int col, int p, int buf) {
+        *reinterpret_cast<u32x2 *>(lds + wb + uint32_t(col) * 2048u + uint32_t(p) * kPart + uint32_t(buf) * kStageB) =
+            u32x2{parts[1][p][2 * col], parts[1][p][2 * col + 1]};
+    };
+    // Read r of a half-stage's nine, in the order the products take them.
+    auto read_operand = [&](int r, int half, int buf, Operands &o) {
+        constexpr int kPartOf[9] = {2, 0, 0, 0, 2, 2, 1, 1, 1}, kBlock[9] = {-1, 0, 1, -1, 0, 1, -1, 0, 1};
+        const int p = kPartOf[r], j = kBlock[r];
+        const uint32_t from = (j < 0 ? ra[half] : rb[half] + uint32_t(j) * 2048u) + uint32_t(p) * kPart +
+                              uint32_t(buf) * kStageB;
+        (j < 0 ? o.a[p] : o.b[j][p]) = *reinterpret_cast<const bf16x8 *>(lds + from);
+    };
+    auto publish = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
 
-    f32x16 acc[TM][2], part[TM][2];
+    // Prologue: stage 0 whole and the A chunk of stage 1 converted; A of
+    // stages 2 and 3 and B of stages 1 and 2 in flight.
+    auto fetch_a = [&](int set) {
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+        for (int x = 0; x < 2; ++x) load_a(set, x);
+    };
+    auto fetch_b = [&](int set) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int e = 0; e < 4; ++e) load_b(set, e);
+    };
+    auto convert_a = [&](int set, int buf) {
 #pragma unroll
-            for (int v = 0; v < 16; ++v) acc[i][j][v] = part[i][j][v] = 0.f;
+        for (int x = 0; x < 12; ++x) convert(0, set, x / 3, x % 3);
+#pragma unroll
+        for (int p = 0; p < kParts; ++p) write_a(p, buf);
+    };
+    auto convert_b = [&](int set, int buf) {
+#pragma unroll
+        for (int x = 0; x < 12; ++x) convert(1, set, x / 3, x % 3);
+#pragma unroll
+        for (int p = 0; p < kParts; ++p) {
+            write_b(0, p, buf);
+            write_b(1, p, buf);
+        }
+    };
+    if (tid == 0) tiny = 0;
+    fetch_a(0);
+    fetch_b(0);
+    fetch_a(1);
+    fetch_b(1);
+    convert_a(0, 0);
+    fetch_a(0);
+    convert_b(0, 0);
+    fetch_b(0);
+    convert_a(1, 1);
+    fetch_a(1);
+    publish();
+    Operands cur;
+#pragma unroll
+    for (int r = 0; r < 9; ++r) read_operand(r, 0, 0, cur);
 
-    // The tile at (m0, n0): row 8(v >> 2) + (v & 3) + 32i of the lane's rows.
-    // The origin passes through an empty asm so that no address is computed
-    // ahead of the branch that stores (it would hold the addresses in
-    // registers over the K loop).
-    auto store = [&](int m0, int n0) {
-        m0 = uniform(m0);
-        n0 = uniform(n0);
-        asm volatile("" : "+s"(m0), "+s"(n0));
-        const size_t tile = size_t(m0) * size_t(N) + n0;
+    f32x16 acc[2] = {}, part[2] = {};
+
+    // One half-stage: twelve MFMAs. HALF 0 multiplies k 0-15 of stage g (buffer
+    // P), reads k 16-31 and converts B of stage g + 1 into buffer P ^ 1; HALF
+    // 1 multiplies k 16-31, reads k 0-15 of stage g + 1 and converts A of stage
+    // g + 2 into buffer P, which no wave reads any more.
+    auto half_stage = [&](auto hc, auto pc, auto sc) __attribute__((always_inline)) {
+        constexpr int HALF = decltype(hc)::value, P = decltype(pc)::value;
+        constexpr bool START = decltype(sc)::value;
+        constexpr int set = HALF == 0 ? P ^ 1 : P, out = set;
+        Operands nxt;
+        if constexpr (HALF == 1) publish();
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+        for (int n = 0; n < 12; ++n) {
+            const int p = n >> 1, j = n & 1;
+            __builtin_amdgcn_sched_barrier(0);
+            if (START && p == 0) {
+                acc[j] += part[j];
+                part[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.a[kPartA[p]], cur.b[j][kPartB[p]], f32x16{}, 0, 0, 0);
+            } else {
+                part[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur.a[kPartA[p]], cur.b[j][kPartB[p]], part[j], 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (n < 9) read_operand(n, HALF ^ 1, HALF == 0 ? P : P ^ 1, nxt);
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const size_t at = tile + size_t(i * 32 + 8 * (v >> 2) + (v & 3)) * size_t(N) + out_lane;
-                const float x0 = acc[i][0][v], x1 = acc[i][1][v];
-                if constexpr (PAIRS) {
-                    *reinterpret_cast<float2 *>(C + at) = make_float2(x0, x1);
-                    if (sum) {  // block-uniform
-                        const float2 r = *reinterpret_cast<const float2 *>(residual + at);
-                        *reinterpret_cast<float2 *>(sum + at) = make_float2(x0 + r.x, x1 + r.y);
-                    }
-                } else {
-                    C[at] = x0;
-                    C[at + 1] = x1;
-                    if (sum) {
-                        sum[at] = x0 + residual[at];
-                        sum[at + 1] = x1 + residual[at + 1];
+            for (int x = 0; x < 12; ++x) {
+                if (x * 10 / 12 != n) continue;
+                const int u = x / 3, piece = x % 3;
+                convert(HALF == 0, set, u, piece);
+                if (piece == 2) {
+                    if (HALF == 0) {
+                        if (u == 2) {
+                            load_b(set, 0);
+                            load_b(set, 1);
+                        }
+                        if (u == 3) {
+                            load_b(set, 2);
+                            load_b(set, 3);
+                        }
+                        if (u & 1)
+#pragma unroll
+                            for (int w = 0; w < kParts; ++w) write_b(u >> 1, w, out);
+                    } else {
+                        if (u & 1) load_a(set, u >> 1);
+                        if (u == 3)
+#pragma unroll
+                            for (int w = 0; w < kParts; ++w) write_a(w, out);
                     }
                 }
             }
-    };
-
-    bases(0, da, db);
-    bases(mine > 1 ? 1 : 0, nda, ndb);
-    issue_next(0);
-    issue_next(1);
-    issue_next(2);
-    wait_loads_barrier<2 * kLoads>();
-    Quarter<TM> cur;
-    read_quarter(0, 0, cur);
-    int m0, n0, pm0 = 0, pn0 = 0;
-    tile_origin(0, m0, n0);
-
-    // One stage at position U of an eight-stage iteration. Every stage issues
-    // kLoads loads (stage g + 3 of the sequence, or, past its end, data that
-    // is never read), so the wait for stage g + 1 is always vmcnt(kLoads),
-    // except after FIRST: the first iteration of a tile after another one
-    // stores that tile at the end of its stage U = 0, and vmcnt counts those
-    // stores too, so stage U = 1 waits for everything.
-    auto stage = [&](auto uc, auto fc) __attribute__((always_inline)) {
-        constexpr int U = decltype(uc)::value;
-        constexpr bool FIRST = decltype(fc)::value;
-        constexpr int slot = U % kDepth;
-        constexpr bool run_start = U % kFoldRun == 0;
-        wait_loads_barrier<(FIRST && U == 1) ? 0 : kLoads>();  // publishes stage g + 1
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            Quarter<TM> nxt;
-            const int rslot = q < 3 ? slot : (slot + 1) % kDepth, rq = (q + 1) % 4;
             __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int i = 0; i < TM; ++i)
-#pragma unroll
-                    for (int j = 0; j < 2; ++j) {
-                        const int n = (e * TM + i) * 2 + j;  // MFMA index in the quarter
-                        const float b = j ? cur.b[e].y : cur.b[e].x;
-                        if (run_start && q == 0 && e == 0) {
-                            // Fold the previous run's sums of this block, then
-                            // restart it from zero.
-                            acc[i][j] += part[i][j];
-                            part[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(cur.a[i][e], b, f32x16{}, 0, 0, 0);
-                            __builtin_amdgcn_sched_barrier(0);
-                        } else {
-                            part[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(cur.a[i][e], b, part[i][j], 0, 0, 0);
-                        }
-                        // The next quarter's reads go out one after each of
-                        // this quarter's first MFMAs, pinned there (the
-                        // scheduler would sink them to their use to save
-                        // registers); issued back to back they waited on the
-                        // LDS pipe beside the LDS-direct writes.
-                        if (n < TM + 4) {
-                            __builtin_amdgcn_sched_barrier(0);
-                            read_part(rslot, rq, n, nxt);
-                            __builtin_amdgcn_sched_barrier(0);
-                        }
-                        // A load goes out after MFMA 6 of each eight, one
-                        // before the group's end: 4096^3 920.8 -> 913.5 us
-                        // against the group's last MFMA (after MFMA 5 917.4,
-                        // 4 917.8, 3 921.2, 0 919.5). Moving the operand
-                        // reads instead (one MFMA later, spread over the
-                        // quarter, or B rows first) changed nothing (0.2%).
-                        if (n % 8 == 6) {
-                            __builtin_amdgcn_sched_barrier(0);
-                            issue_part((U + 3) % kDepth, q * (kMfmas / 8) + n / 8);
-                            __builtin_amdgcn_sched_barrier(0);
-                        }
-                    }
-            __builtin_amdgcn_sched_barrier(0);
-            cur = nxt;
         }
-        if constexpr (FIRST && U == 0) {
-            store(pm0, pn0);
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j) acc[i][j] = f32x16{};
-        }
+        cur = nxt;
     };
-    auto iteration = [&](auto fc) __attribute__((always_inline)) {
-        stage(std::integral_constant<int, 0>{}, fc);
-        stage(std::integral_constant<int, 1>{}, fc);
-        stage(std::integral_constant<int, 2>{}, fc);
-        stage(std::integral_constant<int, 3>{}, fc);
-        stage(std::integral_constant<int, 4>{}, fc);
-        stage(std::integral_constant<int, 5>{}, fc);
-        stage(std::integral_constant<int, 6>{}, fc);
-        stage(std::integral_constant<int, 7>{}, fc);
+    auto stage = [&](auto pc, auto sc) __attribute__((always_inline)) {
+        half_stage(std::integral_constant<int, 0>{}, pc, sc);
+        half_stage(std::integral_constant<int, 1>{}, pc, std::false_type{});
+    };
+    const std::integral_constant<int, 0> even{};
+    const std::integral_constant<int, 1> odd{};
+
+    // Output row 8 (v >> 2) + (v & 3) of the lane's rows, columns 2c, 2c + 1
+    // of the wave's (DUAL: column c of each product).
+    const uint32_t out_lane = uint32_t((wm * 32 + 4 * h) * N + (DUAL ? wn * 32 + c : wn * 64 + 2 * c));
+    auto store = [&](int m0, int n0) {
+        m0 = uniform(m0);
+        n0 = uniform(n0);
+        // No address is computed ahead of the K loop, which would hold the
+        // sixteen rows' offsets in registers across it.
+        uint32_t from = out_lane, row = uint32_t(N);
+        asm volatile("" : "+s"(m0), "+s"(n0), "+s"(row), "+v"(from));
+        const size_t tile = size_t(m0) * row + n0;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            const size_t o = tile + size_t(8 * (v >> 2) + (v & 3)) * row + from;
+            const float x0 = acc[0][v], x1 = acc[1][v];
+            if constexpr (DUAL) {
+                C[o] = x0;
+                C2[o] = x1;
+                sum[o] = swiglu(x0, x1);
+            } else if constexpr (FORM == RingForm::Pairs) {
+                *reinterpret_cast<float2 *>(C + o) = make_float2(x0, x1);
+                if (sum) {  // block-uniform
+                    const float2 r = *reinterpret_cast<const float2 *>(residual + o);
+                    *reinterpret_cast<float2 *>(sum + o) = make_float2(x0 + r.x, x1 + r.y);
+                }
+            } else {
+                C[o] = x0;
+                C[o + 1] = x1;
+                if (sum) {
+                    sum[o] = x0 + residual[o];
+                    sum[o + 1] = x1 + residual[o + 1];
+                }
+            }
+        }
     };
 
-    for (int j = 0; j < mine; ++j) {
-        if (j > 0) {
-            pm0 = m0;
-            pn0 = n0;
-            tile_origin(j, m0, n0);
-            // The cursor is in tile j now; its wrap goes to tile j + 1.
-            bases(j + 1 < mine ? j + 1 : j, nda, ndb);
-            iteration(std::true_type{});
-        } else {
-            iteration(std::false_type{});
+    // The wave's outputs of the tile at (m0, n0) again, in FP32 from global
+    // memory: lane (h, c) takes k 4h on of every eight, for A row c and B
+    // columns 2c, 2c + 1 (DUAL: column c of each product).
+    auto again = [&](int m0, int n0) __attribute__((always_inline)) {
+        const float *a = A + size_t(m0 + 32 * wm + c) * size_t(K) + 4 * h;
+        const size_t col = size_t(4 * h) * size_t(N) + n0 + (DUAL ? 32 * wn + c : 64 * wn + 2 * c);
+        const float *b0 = B + col, *b1 = DUAL ? B2 + col : B + col + 1;
+        f32x16 run[2] = {};
+        acc[0] = acc[1] = f32x16{};
+        for (int k = 0; k < K; k += 8) {
+            const f32x4 x = *reinterpret_cast<const f32x4 *>(a + k);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const size_t row = size_t(k + e) * size_t(N);
+                run[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], b0[row], run[0], 0, 0, 0);
+                run[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], b1[row], run[1], 0, 0, 0);
+            }
+            if ((k & 127) == 120) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    acc[j] += run[j];
+                    run[j] = f32x16{};
+                }
+            }
         }
-        for (int it = 1; it < nk / kUnroll; ++it) iteration(std::false_type{});
+    };
+
+    bool was_tiny = false;
+    for (int t = 0; t < mine; ++t) {
+        if (t > 0) aim_next(t + 1);
+        for (int it = 0; it < nk / kUnroll; ++it) {
+            stage(even, std::true_type{});
+            stage(odd, std::false_type{});
+            for (int r = 1; r < kUnroll / 2; ++r) {
+                stage(even, std::false_type{});
+                stage(odd, std::false_type{});
+            }
+        }
+        int m0, n0;
+        tile_origin(t, m0, n0);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            acc[j] += part[j];
+            part[j] = f32x16{};
+        }
+        // The conversions of up to two stages of the next tile are in
+        // `smallest` too, so a tile also counts as tiny when the one before it
+        // did. All waves have read the flag when the second barrier opens; the
+        // stages of the next tile lie between its clearing and its next use.
+        if (__any(lossy(smallest)) && lane == 0) tiny = 1;
+        smallest = u16x2{0xffff, 0xffff};
+        publish();
+        const bool is_tiny = uniform(tiny) != 0;
+        publish();
+        if (tid == 0) tiny = 0;
+        float total = 0.f;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) total += acc[0][v] * 0.f + acc[1][v] * 0.f;  // 0, or NaN
+        if (is_tiny || was_tiny || __any(total != 0.f)) again(m0, n0);
+        was_tiny = is_tiny;
+        store(m0, n0);
+        acc[0] = acc[1] = f32x16{};
     }
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] += part[i][j];
-    store(m0, n0);
-    // Loads past the sequence's end are still in flight; LDS must not be
-    // released under them.
-    drain_vmem();
 }
-
-// Eight waves of 32x64 (two per SIMD) against four of 64x64: 149.3 against
-// 147.4 TFLOP/s at 4096^3, 146.4 against 144.7 at 4096x11008x4096, with the
-// interleaved operand reads (bit-identical outputs).
-constexpr int kRingTM = 1;
-static_assert(512 / kRingTM == ring::kThreads, "the launch's workgroup size");
 
 }  // namespace
 
 hipError_t launch_gemm_ring(hipStream_t stream, const float *a, const float *b, float *c, uint32_t n, uint32_t k,
                             int tiles_m, int tiles_n, unsigned grid, const float *residual, float *sum) {
-    constexpr int TM = kRingTM;
-    const dim3 block(512 / TM);
+    const dim3 block(ring::kThreads);
     const bool pairs = ((reinterpret_cast<uintptr_t>(c) | reinterpret_cast<uintptr_t>(residual) |
                          reinterpret_cast<uintptr_t>(sum)) & 7u) == 0;
     if (pairs)
-        hipLaunchKernelGGL((gemm_f32_ring<TM, true>), dim3(grid), block, 0, stream, a, b, c, int(n), int(k), tiles_m,
-                           tiles_n, residual, sum);
+        hipLaunchKernelGGL((gemm_f32_ring<RingForm::Pairs>), dim3(grid), block, 0, stream, a, b, nullptr, c, nullptr,
+                           int(n), int(k), tiles_m, tiles_n, residual, sum);
     else
-        hipLaunchKernelGGL((gemm_f32_ring<TM, false>), dim3(grid), block, 0, stream, a, b, c, int(n), int(k), tiles_m,
-                           tiles_n, residual, sum);
+        hipLaunchKernelGGL((gemm_f32_ring<RingForm::Plain>), dim3(grid), block, 0, stream, a, b, nullptr, c, nullptr,
+                           int(n), int(k), tiles_m, tiles_n, residual, sum);
+    return hipGetLastError();
+}
+
+hipError_t launch_gemm_ring_swiglu(hipStream_t stream, const float *a, const float *bg, const float *bu, float *g,
+                                   float *u, float *act, uint32_t n, uint32_t k, int tiles_m, int tiles_n,
+                                   unsigned grid) {
+    hipLaunchKernelGGL((gemm_f32_ring<RingForm::Dual>), dim3(grid), dim3(ring::kThreads), 0, stream, a, bg, bu, g, u,
+                       int(n), int(k), tiles_m, tiles_n, nullptr, act);
     return hipGetLastError();
 }
 

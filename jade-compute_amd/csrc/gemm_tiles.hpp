@@ -13,18 +13,17 @@ namespace hipk {
 // checks before it routes a product there.
 namespace ring {
 constexpr int kBM = 128, kBN = 128;
-constexpr int kDepth = 4;   // 32-deep stages resident in LDS
-constexpr int kUnroll = 8;  // stages per loop iteration; K must be a multiple of 32 * kUnroll
+constexpr int kUnroll = 8;     // stages per loop iteration; K must be a multiple of 32 * kUnroll
 constexpr int kThreads = 512;  // eight waves of 32x64
-// Stages summed in MFMA accumulators before each fold: eight, where the tile
-// loops fold every four. Against four: 4096^3 928 -> 920 us (+0.8%),
-// 4096x11008x4096 2648 -> 2620, 4096x1024x2816 164.4 -> 162.9; the worst
-// 4096^3 output then uses a third of the 1e-4 + 1e-4|e| tolerance (a fifth
-// with four).
-constexpr int kFoldRun = 8;
-constexpr uint32_t kAStageB = kBM * 32 * 4, kBStageB = 32 * kBN * 4;  // 16 KiB each
-constexpr uint32_t kBRegion = kDepth * kAStageB;                      // B stages from 64 KiB
-constexpr uint32_t kLdsBytes = kDepth * (kAStageB + kBStageB);        // 128 KiB
+// Stages summed in the MFMA accumulators before each fold (the loop's
+// iteration). A run of 256 k leaves 2.5e-7 of relative error at 4096^3, one of
+// 128 k 2.0e-7, one of 1024 k 4.9e-7.
+constexpr int kFoldRun = kUnroll;
+constexpr uint32_t kPart = 128 * 32 * 2;          // one bf16 part of an A or B stage: 8 KiB
+constexpr uint32_t kBRegion = 3 * kPart;          // B parts from 24 KiB of a stage
+constexpr uint32_t kStageB = 6 * kPart;           // 48 KiB
+constexpr uint32_t kStages = 2 * kStageB;         // 96 KiB
+constexpr uint32_t kLdsBytes = kStages + 4;       // with the tile's flag
 }  // namespace ring
 
 // C = A B on the persistent kernel: `grid` workgroups (at most one per CU)
@@ -33,6 +32,11 @@ constexpr uint32_t kLdsBytes = kDepth * (kAStageB + kBStageB);        // 128 KiB
 hipError_t launch_gemm_ring(hipStream_t stream, const float *a, const float *b, float *c, uint32_t n, uint32_t k,
                             int tiles_m, int tiles_n, unsigned grid, const float *residual = nullptr,
                             float *sum = nullptr);
+// g = a bg, u = a bu, act = swiglu(g, u) on the same kernel over a tiles_m x
+// tiles_n grid of 128x64 tiles of each product.
+hipError_t launch_gemm_ring_swiglu(hipStream_t stream, const float *a, const float *bg, const float *bu, float *g,
+                                   float *u, float *act, uint32_t n, uint32_t k, int tiles_m, int tiles_n,
+                                   unsigned grid);
 
 namespace {
 
