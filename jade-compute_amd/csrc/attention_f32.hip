@@ -20,6 +20,14 @@
 // head share one XCD (workgroups go round-robin over 8 XCDs by linear id). A
 // wave skips 32-key sub-tiles that lie wholly above its causal diagonal.
 //
+// Whole rows of 16-byte multiples run on bf16 parts instead
+// (attention_flash.hip); this kernel takes other head dims, and the split
+// launches, where the parts gain nothing: a slice is a few tiles, and the flash
+// kernel's prologue (two tiles loaded and split before the first product)
+// weighs as much (us, this kernel and that one: H2 S1024 D64 causal 16.0 / 16.9,
+// H1 S700 D128 causal 20.7 / 24.8, H2 S513 D32 11.0 / 12.4, H1 S2048 D64 21.9 /
+// 21.4).
+//
 // Grids too small to fill the chip (fewer blocks than CUs) split each block's
 // key tiles into slices of `per` tiles, one block per live slice. A slice writes its
 // unnormalised O, running max and normaliser to a workspace, and
@@ -27,6 +35,7 @@
 // O = sum_z 2^(m_z - M) O_z / sum_z 2^(m_z - M) l_z with M = max_z m_z.
 // Fixed-size slices give a causal grid's long rows more slices than its short
 // ones, so every live slice costs about the same.
+#include "attention_flash.hpp"
 #include "kernels.hpp"
 
 #include <algorithm>
@@ -666,13 +675,29 @@ void launch_combine(hipStream_t stream, const float *part, const float2 *ml, flo
                            c);
 }
 
+// Rows of 16-byte multiples in heads below 2 GiB (the K and V loads are buffer
+// loads over one head) run on bf16 parts (attention_flash.hip).
+bool on_parts(uint32_t seq, uint32_t dim) {
+    return dim % 4 == 0 && uint64_t(seq) * uint64_t(dim) * 4u < (uint64_t(1) << 31);
+}
+
 int padded_dim(uint32_t dim) { return dim <= 32 ? 32 : dim <= 64 ? 64 : 128; }
 
-// Eight waves per block when that still gives at least two blocks per CU;
-// four waves (128 queries) for small problems so more CUs get work.
-int waves_for(uint32_t heads, uint32_t seq) {
-    const uint64_t blocks8 = uint64_t(heads) * ((seq + 255) / 256);
-    return blocks8 >= 512 ? 8 : 4;
+// Waves per block of an unsplit launch (32 queries each): four, or eight where
+// the flash kernel on bf16 parts then finishes first. At head dims over 64 it
+// runs two waves per SIMD with eight and one with four, and a CU takes 1.62
+// times as long for 256 queries with four (H64 S2048 noncausal: D128 768 us
+// against 641, D96 633 against 505, both in whole rounds of the CUs).
+// Noncausal blocks are alike, so whole rounds decide; causal rows of unequal
+// length fill the rounds, and eight waves take grids of at least two rounds.
+// Rows without 16-byte multiples run the FP32 kernel, which takes eight waves
+// in the same causal case and at every head dim.
+int waves_for(uint32_t heads, uint32_t seq, uint32_t dim, bool causal) {
+    const uint64_t blocks4 = uint64_t(heads) * ((seq + 127) / 128), blocks8 = uint64_t(heads) * ((seq + 255) / 256);
+    const auto rounds = [](uint64_t blocks) { return (blocks + 255) / 256; };
+    if (!on_parts(seq, dim)) return blocks8 >= 512 ? 8 : 4;
+    if (dim <= 64 || blocks4 < 256) return 4;
+    return (causal ? blocks8 >= 512 : 100 * rounds(blocks8) < 62 * rounds(blocks4)) ? 8 : 4;
 }
 
 constexpr uint32_t kCUs = 256;
@@ -687,7 +712,7 @@ struct SplitPlan {
 // shortest slices whose live count still fits one block per CU, so the whole
 // launch is one round of equal-cost slices (at most 16 slices per row).
 SplitPlan split_plan(uint32_t heads, uint32_t seq, bool causal) {
-    const uint32_t bq = 32u * uint32_t(waves_for(heads, seq));
+    constexpr uint32_t bq = 128;  // small grids take four-wave blocks
     const uint32_t q_blocks = (seq + bq - 1) / bq;
     const uint32_t max_tiles = (seq + kBKV - 1) / kBKV;
     if (uint64_t(heads) * q_blocks >= kCUs) return {max_tiles, 1, 0};
@@ -1288,14 +1313,21 @@ hipError_t launch_online(hipStream_t stream, const float *q, const float *k, con
     using S = AttnShape<DP, NW>;
     const unsigned q_blocks = (seq + S::kBQ - 1) / S::kBQ;
     const float qscale = (1.0f / sqrtf(float(dim))) * kLog2e;
+    if constexpr (!SPLIT)
+        if (vec && on_parts(seq, dim))
+            return launch_attention_flash(stream, FlashArgs{q, k, v, out, heads, seq, dim, CAUSAL, qscale, NW});
     const dim3 grid = SPLIT ? dim3(plan.live) : dim3(heads, q_blocks), block(S::kThreads);
-    // The vector kernel reads K and V through buffer loads over one head.
-    if (vec && uint64_t(seq) * uint64_t(dim) * 4u < (uint64_t(1) << 31))
-        hipLaunchKernelGGL((attention_online_mfma<DP, NW, CAUSAL, true, SPLIT>), grid, block, 0, stream, q, k, v,
-                           out, ml, int(seq), int(dim), qscale, int(plan.per), int(heads));
-    else
-        hipLaunchKernelGGL((attention_online_mfma<DP, NW, CAUSAL, false, SPLIT>), grid, block, 0, stream, q, k, v,
-                           out, ml, int(seq), int(dim), qscale, int(plan.per), int(heads));
+    // Split launches of 16-byte rows read K and V through buffer loads over one
+    // head; whole rows of 16 bytes took the flash kernel above.
+    if constexpr (SPLIT) {
+        if (vec && on_parts(seq, dim)) {
+            hipLaunchKernelGGL((attention_online_mfma<DP, NW, CAUSAL, true, SPLIT>), grid, block, 0, stream, q, k, v,
+                               out, ml, int(seq), int(dim), qscale, int(plan.per), int(heads));
+            return hipGetLastError();
+        }
+    }
+    hipLaunchKernelGGL((attention_online_mfma<DP, NW, CAUSAL, false, SPLIT>), grid, block, 0, stream, q, k, v, out, ml,
+                       int(seq), int(dim), qscale, int(plan.per), int(heads));
     return hipGetLastError();
 }
 
@@ -1376,8 +1408,7 @@ hipError_t dispatch_dim(hipStream_t stream, const float *q, const float *k, cons
     }
     const SplitPlan plan = split_plan(heads, seq, causal);
     if (plan.slices > 1) {
-        // Split grids are small grids, which always take four-wave blocks.
-        if (waves_for(heads, seq) != 4 || workspace == nullptr) return hipErrorInvalidValue;
+        if (workspace == nullptr) return hipErrorInvalidValue;
         float *part = workspace;
         float2 *ml = reinterpret_cast<float2 *>(workspace + split_part_floats(heads, seq, dim, plan.slices));
         const hipError_t status =
@@ -1392,7 +1423,7 @@ hipError_t dispatch_dim(hipStream_t stream, const float *q, const float *k, cons
         return hipGetLastError();
     }
     const SplitPlan whole{plan.per, 1, 0};
-    if (waves_for(heads, seq) == 8)
+    if (waves_for(heads, seq, dim, causal) == 8)
         return causal ? launch_online<DP, 8, true, false>(stream, q, k, v, out, nullptr, heads, seq, dim, whole, vec)
                       : launch_online<DP, 8, false, false>(stream, q, k, v, out, nullptr, heads, seq, dim, whole, vec);
     return causal ? launch_online<DP, 4, true, false>(stream, q, k, v, out, nullptr, heads, seq, dim, whole, vec)
@@ -1420,11 +1451,12 @@ LaunchShape attention_online_shape(uint32_t heads, uint32_t seq, uint32_t dim, b
                 {uint32_t(pairs_waves(dp) * 64), 1, 1},
                 uint32_t(pairs_waves(dp) * 2 * pairs::kUnit * ((dp + 4) * sizeof(float) + sizeof(float2)))};
     }
-    const int nw = waves_for(heads, seq);
+    const int nw = waves_for(heads, seq, dim, causal);
     const uint32_t bq = 32u * nw;
     const SplitPlan plan = split_plan(heads, seq, causal);
     const uint32_t splits = plan.slices;
-    const uint32_t lds = dp == 32 ? lds_bytes<32>(nw) : dp == 64 ? lds_bytes<64>(nw) : lds_bytes<128>(nw);
+    const uint32_t lds = splits <= 1 && on_parts(seq, dim) ? attention_flash_lds_bytes(dim, nw)
+                         : dp == 32 ? lds_bytes<32>(nw) : dp == 64 ? lds_bytes<64>(nw) : lds_bytes<128>(nw);
     static const char *const names[2][3] = {
         {"attention_online_mfma_d32", "attention_online_mfma_d64", "attention_online_mfma_d128"},
         {"attention_online_mfma_d32_split", "attention_online_mfma_d64_split", "attention_online_mfma_d128_split"}};

@@ -87,3 +87,85 @@ def test_persistent_gate_up_special_values(runtime, name):
         t.free()
     check(got_g, a, b, k)
     check(got_u, a, np.ascontiguousarray(b[:, ::-1]), k)
+
+
+def attend(runtime, heads, seq, dim, causal, q, k, v):
+    kernel = runtime.compile({"op": "attention_online", "heads": heads, "seq": seq, "dim": dim, "causal": causal})
+    print(f"attention H{heads} S{seq} D{dim} causal {causal}: {kernel.launch}", flush=True)
+    bufs = [runtime.resident(x) for x in (q, k, v)] + [runtime.alloc(heads * seq * dim)]
+    runtime.execute([(kernel, bufs)], 2)
+    got = runtime.download(bufs[3])
+    for x in bufs:
+        x.free()
+    return got, kernel.launch
+
+
+@pytest.mark.parametrize("heads,seq,dim,causal,threads", [
+    (24, 1531, 80, False, 512),  # eight waves: one round of 144 blocks against two of 288
+    (33, 1020, 128, False, 512), (33, 1020, 128, True, 256),  # heads not a multiple of the XCDs
+    (256, 300, 72, True, 512), (171, 513, 128, True, 512),  # eight waves, causal
+    (32, 1024, 100, True, 256), (32, 1000, 96, True, 256),  # four waves, one per SIMD
+    (40, 900, 64, True, 256), (9, 3700, 20, False, 256),  # head dims to 64 and 32
+    (304, 1, 64, False, 256), (304, 33, 96, True, 256), (304, 31, 128, False, 256), (272, 32, 4, True, 256),
+    (272, 129, 36, False, 256),  # one key; the edges of a tile; one block and a row more
+])
+def test_flash_on_parts_shapes(runtime, heads, seq, dim, causal, threads):
+    n = heads * seq * dim
+    q, k, v = orc.normal(n, 0x81), orc.normal(n, 0x82), orc.normal(n, 0x83)
+    got, launch = attend(runtime, heads, seq, dim, causal, q, k, v)
+    assert launch["block"][0] == threads and "split" not in launch["kernel"], launch
+    want = orc.attention_reference(heads, seq, dim, causal, q, k, v)
+    # FP32 rounding of scores of a few units and of sums of weights: 1e-5 of the unit-sized values.
+    assert orc.compare(got, want, 1e-5, 1e-5).status == 0
+
+
+FLASH = [(32, 1000, 96, True), (24, 1531, 80, False), (40, 900, 64, True)]  # four waves, eight, two a SIMD
+
+
+@pytest.mark.parametrize("heads,seq,dim,causal", FLASH)
+def test_flash_on_parts_scaled_operands(runtime, heads, seq, dim, causal):
+    # Operands at the ends of the FP32 range whose scores are ordinary, and
+    # values of V near the smallest normals: as FP32 arithmetic has them.
+    n = heads * seq * dim
+    q, k, v = orc.normal(n, 0x91), orc.normal(n, 0x92), orc.normal(n, 0x93)
+    for sq, sk, sv in ((1e30, 1e-30, 1.0), (1e-30, 1e30, 1.0), (1.0, 1.0, 1e-36)):
+        a, b, c = (np.asarray(x * np.float32(s), np.float32) for x, s in ((q, sq), (k, sk), (v, sv)))
+        got, _ = attend(runtime, heads, seq, dim, causal, a, b, c)
+        want = orc.attention_reference(heads, seq, dim, causal, a, b, c)
+        assert orc.compare(got / np.float32(sv), np.asarray(want) / sv, 2e-5, 2e-5).status == 0, (sq, sk, sv)
+
+
+@pytest.mark.parametrize("heads,seq,dim,causal", FLASH)
+def test_flash_on_parts_non_finite(runtime, heads, seq, dim, causal):
+    n = heads * seq * dim
+    q, k, v = (orc.normal(n, s).reshape(heads, seq, dim).copy() for s in (0xA1, 0xA2, 0xA3))
+    key = seq // 2
+    q[1, :, 0] = np.abs(q[1, :, 0]) + 0.5
+    k[1, key] = 0
+    k[1, key, 0] = -np.inf  # scores of -inf: the key has no weight
+    v[2, key, 3] = np.inf
+    q[3, key, 1] = np.nan
+    got, _ = attend(runtime, heads, seq, dim, causal, q.ravel(), k.ravel(), v.ravel())
+    got = got.reshape(heads, seq, dim)
+    want = np.asarray(orc.attention_reference(heads, seq, dim, causal, *(np.where(np.isfinite(x), x, 0).ravel()
+                                                                       for x in (q, k, v)))).reshape(heads, seq, dim)
+    clean = [h for h in range(heads) if h not in (1, 2, 3)]
+    assert orc.compare(got[clean].ravel(), want[clean].ravel(), 1e-5, 1e-5).status == 0
+    # Head 1: finite everywhere, and what the other keys give.
+    rows = [0, key - 1, key, seq - 1]
+    for r in rows:
+        keys = np.arange(r + 1 if causal else seq)
+        keys = keys[keys != key] if len(keys) > 1 else keys
+        s = q[1, r].astype(np.float64) @ k[1, keys].astype(np.float64).T / np.sqrt(dim)
+        w = np.exp(s - s.max())
+        np.testing.assert_allclose(got[1, r], (w / w.sum()) @ v[1, keys].astype(np.float64), rtol=2e-5, atol=2e-5)
+    assert np.isfinite(got[1]).all()
+    # Head 2: column 3 of every query that weighs the key, the other columns as they were.
+    first = key if causal else 0
+    assert not np.isfinite(got[2, first:, 3]).any()
+    other = [d for d in range(dim) if d != 3]
+    assert orc.compare(got[2][:, other].ravel(), want[2][:, other].ravel(), 1e-5, 1e-5).status == 0
+    # Head 3: the one query.
+    assert np.isnan(got[3, key]).all()
+    rest = [r for r in range(seq) if r != key]
+    assert orc.compare(got[3, rest].ravel(), want[3, rest].ravel(), 1e-5, 1e-5).status == 0
