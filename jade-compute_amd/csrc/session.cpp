@@ -30,7 +30,12 @@ Session::Session(int ordinal) {
         // Default priority on purpose: every queue of this library runs at the
         // same priority.
         expect(hipStreamCreateWithFlags(&queue_, hipStreamNonBlocking), "creating the session queue");
-        expect(hipEventCreate(&clock_[0]), "creating the start event");
+        // The start event only takes a time: work before it has been waited for,
+        // and the kernels after it acquire for themselves. Without a system
+        // fence of its own a call of one near-empty kernel takes 12.1 us
+        // instead of 15.4 (launch and wait alone: 10.9). The stop event keeps
+        // its fence.
+        expect(hipEventCreateWithFlags(&clock_[0], hipEventDisableSystemFence), "creating the start event");
         expect(hipEventCreate(&clock_[1]), "creating the stop event");
     } catch (...) {
         release_all();
