@@ -42,6 +42,7 @@
 //  * Other shapes with too few output tiles to fill 256 CUs split K over
 //    gridDim.y: each slice writes a partial product to a workspace and a
 //    reduction kernel sums the slices in slice order (deterministic, no atomics).
+#include "gemm_rows16.hpp"
 #include "gemm_tiles.hpp"
 #include "kernels.hpp"
 #include "ops.hpp"
@@ -1850,6 +1851,7 @@ struct Plan {
     int tail_tm, tail_tn;  // big plans: the partial last round's tile, (64*tail_tm) x (64*tail_tn)
     bool bufa;             // direct plans over unaligned A rows: A through buffer loads
     bool ring = false;     // persistent 128x128 tiles, one workgroup per CU (gemm_f32_ring)
+    int rows16 = 0;        // > 0: gemm_f32_rows16 with this many waves (tiles_n counts 32-column tiles)
 };
 
 constexpr int kSlots = 512;        // co-resident 256-thread workgroups: two per CU
@@ -2059,7 +2061,21 @@ bool ring_takes(uint32_t m, uint32_t n, uint32_t k, const Plan &tiles) {
     return 10 * t >= 9 * rounds * uint64_t(kCUs);
 }
 
+// At most 16 rows, K at most 512 and fewer than 64 tiles of 32 columns (more
+// fill the chip as direct-load 32x32 tiles: 16x2048x512 4.8 us there, 5.1
+// here): one launch of four waves (K to 256) or eight a tile. gemm_rows16.hip
+// has the figures of both sides.
+int rows16_waves(uint32_t m, uint32_t n, uint32_t k) {
+    if (m > 16 || k > 512 || (n + 31) / 32 >= 64) return 0;
+    return k <= 256 ? 4 : 8;
+}
+
 Plan plan_for(uint32_t m, uint32_t n, uint32_t k) {
+    if (const int waves = rows16_waves(m, n, k)) {
+        Plan r{1, 1, 1, int(k), 1, int((n + 31) / 32), false, 0, 0, 1, 0, 0};
+        r.rows16 = waves;
+        return r;
+    }
     const Plan p = plan_tiles(m, n, k);
     if (!ring_takes(m, n, k, p)) return p;
     Plan r{2, 2, 1, int(k), int(m / ring::kBM), int(n / ring::kBN), false, 0, 0, 1, 0, 0};
@@ -2221,6 +2237,7 @@ Route route_for(uint32_t m, uint32_t n, uint32_t k) {
         r.launchable = r.launchable && r.vec;  // big_fits / ring_fits imply n % 128 == 0 and k % 32 == 0
         return r;
     }
+    if (p.rows16) return r;
     if (p.direct) {
         r.launchable = r.launchable && (k % 4 == 0 ? (p.slices == 1 || p.direct == 4) : (p.bufa && p.slices == 1));
         return r;
@@ -2314,6 +2331,11 @@ LaunchShape gemm_f32_shape(uint32_t m, uint32_t n, uint32_t k) {
                 {uint32_t(std::min(p.tiles_m * p.tiles_n, kCUs)), 1, 1},
                 {ring::kThreads, 1, 1},
                 ring::kLdsBytes};
+    if (p.rows16)
+        return {p.rows16 == 4 ? "gemm_f32_rows16_w4" : "gemm_f32_rows16_w8",
+                {uint32_t(p.tiles_n), 1, 1},
+                {uint32_t(64 * p.rows16), 1, 1},
+                uint32_t(p.rows16 * 16 * 32 * sizeof(float))};
     if (p.big) {  // the first launch; a partial last round follows as smaller tiles
         const char *name = "gemm_f32_mfma_256x256x32";
         if (p.big_full < p.tiles_m * p.tiles_n)
@@ -2362,7 +2384,7 @@ LaunchShape gemm_f32_shape(uint32_t m, uint32_t n, uint32_t k) {
 
 bool gemm_f32_pairable(uint32_t m, uint32_t n, uint32_t k) {
     const Route r = route_for(m, n, k);
-    return r.launchable && !r.plan.big && !r.plan.ring && !r.plan.direct && r.kg == 1 && r.plan.slices == 1;
+    return r.launchable && !r.plan.big && !r.plan.ring && !r.plan.rows16 && !r.plan.direct && r.kg == 1 && r.plan.slices == 1;
 }
 
 hipError_t gemm_f32_pair(hipStream_t stream, const float *a0, const float *b0, float *c0, const float *a1,
@@ -2387,6 +2409,7 @@ hipError_t gemm_f32_residual(hipStream_t stream, const float *a, const float *b,
     if (r.plan.ring)
         return launch_gemm_ring(stream, a, b, c, n, k, r.plan.tiles_m, r.plan.tiles_n,
                                 unsigned(std::min(r.plan.tiles_m * r.plan.tiles_n, kCUs)), residual, sum);
+    if (r.plan.rows16) return launch_gemm_rows16(stream, r.plan.rows16, a, b, c, m, n, k, residual, sum);
     PairArgs extra{};
     extra.residual = residual;
     extra.sum = sum;
@@ -2453,6 +2476,7 @@ hipError_t gemm_f32(hipStream_t stream, const float *a, const float *b, float *c
         return launch_gemm_ring(stream, a, b, c, n, k, p.tiles_m, p.tiles_n,
                                 unsigned(std::min(p.tiles_m * p.tiles_n, kCUs)));
     }
+    if (p.rows16) return launch_gemm_rows16(stream, p.rows16, a, b, c, m, n, k, nullptr, nullptr);
     if (p.big) {
         hipLaunchKernelGGL(gemm_f32_mfma_256, dim3(unsigned(p.big_full)), dim3(big::kThreads), 0, stream, a, b, c,
                            int(m), int(n), int(k), p.tiles_m, p.tiles_n);

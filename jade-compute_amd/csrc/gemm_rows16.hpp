@@ -1,0 +1,17 @@
+// Host interface of the GEMM for at most 16 rows and short K (gemm_rows16.hip).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+namespace jade {
+namespace hipk {
+
+// C[m,n] = A[m,k] B[k,n], m at most 16, k at most 64 * waves (4 or 8); with
+// `sum` non-null also sum = C + residual. A and B below 2 GiB.
+hipError_t launch_gemm_rows16(hipStream_t stream, int waves, const float *a, const float *b, float *c, uint32_t m,
+                              uint32_t n, uint32_t k, const float *residual, float *sum);
+
+}  // namespace hipk
+}  // namespace jade

@@ -1,0 +1,44 @@
+"""The GEMM for at most 16 rows and short K (csrc/gemm_rows16.hip): edges of
+its slices, columns and waves, any alignment, values past the ends of A and B,
+and the residual Add in its epilogue, against the FP64 oracle."""
+import numpy as np
+import pytest
+
+import oracle_binding as orc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("m,n,k,waves", [
+    (1, 1, 1, 4), (8, 256, 128, 4), (8, 128, 256, 4), (16, 33, 31, 4), (7, 100, 257, 8), (16, 512, 512, 8),
+    (3, 31, 32, 4), (16, 2016, 65, 4), (5, 1999, 511, 8), (15, 64, 129, 4), (2, 30, 33, 4)])
+def test_rows16_shapes(runtime, m, n, k, waves):
+    launch = runtime.compile({"op": "gemm", "m": m, "n": n, "k": k, "tiled": True}).launch
+    assert launch["kernel"] == f"gemm_f32_rows16_w{waves}" and launch["grid"][0] == (n + 31) // 32, launch
+    a, b, x = orc.values(m * k, 0x61, 1.0), orc.values(k * n, 0x62, 1.0), orc.values(m * n, 0x63, 1.0)
+    # The ends of A and B: an Inf in the last column of A's last row and in B's last element stay there.
+    for special in (False, True):
+        if special and (m < 2 or n < 2):
+            continue
+        a2, b2 = a.copy(), b.copy()
+        if special:
+            a2[-1] = np.inf   # A[m-1][k-1]
+            b2[0] = np.nan    # B[0][0]
+        bufs = [runtime.resident(t) for t in (a2, b2, x)] + [runtime.alloc(m * n), runtime.alloc(m * n)]
+        gemm = runtime.compile({"op": "gemm", "m": m, "n": n, "k": k, "tiled": True})
+        add = runtime.compile({"op": "add", "len": m * n})
+        jobs = [(gemm, [bufs[0], bufs[1], bufs[3]]), (add, [bufs[3], bufs[2], bufs[4]])]
+        assert runtime.plan(jobs) == [("gemm_residual", 0)]
+        print(f"rows16 {m}x{n}x{k} special {special}", flush=True)
+        runtime.execute(jobs, 2)
+        got, total = runtime.download(bufs[3]).reshape(m, n), runtime.download(bufs[4]).reshape(m, n)
+        for t in bufs:
+            t.free()
+        want = np.asarray(orc.gemm_reference(m, n, k, a, b)).reshape(m, n)
+        rows, cols = (slice(0, m - 1), slice(1, n)) if special else (slice(0, m), slice(0, n))
+        # K roundings of sums of unit products: 2^-24 K^1.5 is far above what FP32 leaves.
+        tol = 2.0 ** -24 * (k + 8) ** 1.0 * 2
+        assert np.abs(got[rows, cols] - want[rows, cols]).max() <= tol
+        if special:
+            assert np.isnan(got[:, 0]).all() and not np.isfinite(got[m - 1]).any()
+        np.testing.assert_array_equal(total[rows, cols], got[rows, cols] + x.reshape(m, n)[rows, cols])
