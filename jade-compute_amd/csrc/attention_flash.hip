@@ -15,7 +15,7 @@
 // probabilities, and splitting each K and V element once per block. Eight
 // waves share a tile, two per SIMD, so that one wave's softmax runs beside the
 // other's MFMAs. Measured (us) against the FP32-MFMA kernel: H128 S4096 D128
-// causal 4090 -> 2671 (206 TFLOP/s), H64 S2048 D128 noncausal 996 -> 641, H128
+// causal 4100 -> 2575 (214 TFLOP/s), H64 S2048 D128 noncausal 996 -> 641, H128
 // S4096 D64 causal 2238 -> 1466, H24 S1531 D80 noncausal 411 -> 156 (dims pad
 // to 96 instead of 128, and 144 blocks of 256 queries run in one round where
 // 288 of 128 took two), H32 S1000 D96 noncausal 144 -> 84. Error against FP64
@@ -149,7 +149,7 @@ attention_flash(const float *__restrict__ Q, const float *__restrict__ K, const 
                 for (int w = 0; w < kParts; ++w) {
                     const uint32_t k = pack(r.x, r.y);
                     p[w][2 * x + u] = k;
-                    r = f32x2{r.x - low_part(k), r.y - high_part(k)};
+                    r = rest_of(r, k);
                 }
             }
         }
@@ -213,7 +213,7 @@ attention_flash(const float *__restrict__ Q, const float *__restrict__ K, const 
     auto piece_of = [&](uint32_t &out, int piece, f32x2 x) {
         const f32x2 from = piece == 0 ? x : rest;
         out = pack(from.x, from.y);
-        if (piece < 2) rest = f32x2{from.x - low_part(out), from.y - high_part(out)};
+        if (piece < 2) rest = rest_of(from, out);
     };
     auto convert_k = [&](int i, int u, int piece) {
         const f32x4 k = kraw[i][u >> 1];
@@ -522,7 +522,7 @@ attention_flash(const float *__restrict__ Q, const float *__restrict__ K, const 
 #pragma unroll
                 for (int w = 0; w < kParts; ++w) {
                     pw[w][u] = pack(r.x, r.y);
-                    r = f32x2{r.x - low_part(pw[w][u]), r.y - high_part(pw[w][u])};
+                    r = rest_of(r, pw[w][u]);
                 }
             }
             row_sum = row_sum * old_weight + lane_sum;
