@@ -2044,7 +2044,9 @@ Plan plan_tiles(uint32_t m, uint32_t n, uint32_t k);
 // least 512, when the plan it replaces uses 128x128 or 256x256 tiles (those
 // share its tile and its imbalance), or when its grid keeps the CUs busy: the
 // busiest CU holds ceil(t / 256) of the t tiles, at most 1/0.9 of the average.
-// Measured on MI355X against the tile plans (TFLOP/s): 4096^3 141.6 -> 149.3,
+// Measured on MI355X against the tile plans (TFLOP/s), when the persistent
+// kernel ran FP32 MFMAs (on bf16 parts it takes 0.75 to 0.8 of those times; the
+// shapes that lost have not been measured again): 4096^3 141.6 -> 149.3,
 // 4096x11008x4096 138.6 -> 146.4, 5120x5120x2048 127.5 -> 131.9 (256x256
 // tiles and a tail before), 4352x4096x1024 110.4 -> 122.7, 2560^3 109.5 ->
 // 114.6 (400 tiles), 4608^2x1024 117.2 -> 124.1; over 128x64 tiles 2048^3
