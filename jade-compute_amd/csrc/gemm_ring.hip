@@ -48,12 +48,12 @@ namespace {
 // with VALU adds. Error against FP64 (2-norm, relative, uniform [-1, 1)):
 // 4096^3 2.5e-7 (the FP32 MFMAs 3.0e-7), 2048^3 2.4e-7 (3.0e-7).
 //
-// Values the parts do not carry: below 2^-100 the third part meets bf16's
-// smallest subnormal, an infinity minus its own first part is NaN, and at the
-// top of the range the partial products overflow one by one. So every tile
-// that read a nonzero value below 2^-100, and every wave whose sums are not
-// all finite, computes its outputs again from global memory with FP32 MFMAs:
-// infinities, NaN, overflow and tiny operands come out as FP32 arithmetic
+// The operands are scaled before they are split, so that every finite value is
+// carried exactly, subnormals among them (split_bf16.hpp), and the sums are
+// scaled back before they are stored. An infinity minus its own first part is
+// NaN, and scaled values past 2^112 and sums past 2^96 overflow: a wave whose
+// sums are not all finite computes its outputs again from global memory with
+// FP32 MFMAs, so infinities, NaN and overflow come out as FP32 arithmetic
 // gives them, at about a tenth of the speed.
 //
 // Requires M, N multiples of 128 (N of 64 for DUAL), K a multiple of 256,
@@ -97,8 +97,7 @@ __global__ __launch_bounds__(ring::kThreads) __attribute__((amdgpu_waves_per_eu(
     using namespace ring;
     using namespace ring_local;
     constexpr bool DUAL = FORM == RingForm::Dual;
-    __shared__ __attribute__((aligned(1024))) char lds[kStages];
-    __shared__ int tiny;  // whether the tile read a value its parts do not carry
+    __shared__ __attribute__((aligned(1024))) char lds[kLdsBytes];
     const int tid = int(threadIdx.x), lane = tid & 63;
     const int wave = uniform(tid >> 6);
     const int h = lane >> 5, c = lane & 31, wm = wave >> 1, wn = wave & 1;
@@ -185,7 +184,6 @@ __global__ __launch_bounds__(ring::kThreads) __attribute__((amdgpu_waves_per_eu(
     // u / 2, k 2 (u % 2) on), in three pieces.
     uint32_t parts[2][kParts][4];
     f32x2 rest;
-    u16x2 smallest = {0xffff, 0xffff};
     auto convert = [&](int is_b, int set, int u, int piece) {
         if (piece == 0) {
             f32x2 x;
@@ -195,6 +193,7 @@ __global__ __launch_bounds__(ring::kThreads) __attribute__((amdgpu_waves_per_eu(
             } else {
                 x = f32x2{rawa[set][u >> 1][2 * (u & 1)], rawa[set][u >> 1][2 * (u & 1) + 1]};
             }
+            x *= kScale;
             const uint32_t p = pack(x.x, x.y);
             parts[is_b][0][u] = p;
             rest = f32x2{x.x - low_part(p), x.y - high_part(p)};
@@ -204,7 +203,6 @@ __global__ __launch_bounds__(ring::kThreads) __attribute__((amdgpu_waves_per_eu(
             rest = f32x2{rest.x - low_part(p), rest.y - high_part(p)};
         } else {
             parts[is_b][2][u] = pack(rest.x, rest.y);
-            smallest = __builtin_elementwise_min(smallest, doubled_less_one(parts[is_b][0][u]));
         }
     };
     auto write_a = [&](int p, int buf) {
@@ -250,7 +248,6 @@ __global__ __launch_bounds__(ring::kThreads) __attribute__((amdgpu_waves_per_eu(
             write_b(1, p, buf);
         }
     };
-    if (tid == 0) tiny = 0;
     fetch_a(0);
     fetch_b(0);
     fetch_a(1);
@@ -390,7 +387,6 @@ __global__ __launch_bounds__(ring::kThreads) __attribute__((amdgpu_waves_per_eu(
         }
     };
 
-    bool was_tiny = false;
     for (int t = 0; t < mine; ++t) {
         if (t > 0) aim_next(t + 1);
         for (int it = 0; it < nk / kUnroll; ++it) {
@@ -408,21 +404,12 @@ __global__ __launch_bounds__(ring::kThreads) __attribute__((amdgpu_waves_per_eu(
             acc[j] += part[j];
             part[j] = f32x16{};
         }
-        // The conversions of up to two stages of the next tile are in
-        // `smallest` too, so a tile also counts as tiny when the one before it
-        // did. All waves have read the flag when the second barrier opens; the
-        // stages of the next tile lie between its clearing and its next use.
-        if (__any(lossy(smallest)) && lane == 0) tiny = 1;
-        smallest = u16x2{0xffff, 0xffff};
-        publish();
-        const bool is_tiny = uniform(tiny) != 0;
-        publish();
-        if (tid == 0) tiny = 0;
         float total = 0.f;
 #pragma unroll
         for (int v = 0; v < 16; ++v) total += acc[0][v] * 0.f + acc[1][v] * 0.f;  // 0, or NaN
-        if (is_tiny || was_tiny || __any(total != 0.f)) again(m0, n0);
-        was_tiny = is_tiny;
+        acc[0] *= kUnscale;
+        acc[1] *= kUnscale;
+        if (__any(total != 0.f)) again(m0, n0);
         store(m0, n0);
         acc[0] = acc[1] = f32x16{};
     }

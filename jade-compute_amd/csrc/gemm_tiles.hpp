@@ -22,8 +22,7 @@ constexpr int kFoldRun = kUnroll;
 constexpr uint32_t kPart = 128 * 32 * 2;          // one bf16 part of an A or B stage: 8 KiB
 constexpr uint32_t kBRegion = 3 * kPart;          // B parts from 24 KiB of a stage
 constexpr uint32_t kStageB = 6 * kPart;           // 48 KiB
-constexpr uint32_t kStages = 2 * kStageB;         // 96 KiB
-constexpr uint32_t kLdsBytes = kStages + 4;       // with the tile's flag
+constexpr uint32_t kLdsBytes = 2 * kStageB;       // two stages: 96 KiB
 }  // namespace ring
 
 // C = A B on the persistent kernel: `grid` workgroups (at most one per CU)

@@ -59,6 +59,14 @@ __device__ inline f32x2 rest_of(f32x2 x, uint32_t p) {
                  __builtin_amdgcn_fdot2_f32_bf16(part, __builtin_bit_cast(bf16x2, hi), x.y, false)};
 }
 
+// Operands are scaled by kScale before they are split: FP32's smallest
+// subnormal, 2^-149, becomes 2^-133, bf16's, so every finite value splits
+// exactly as long as it stays below 2^112 (v_cvt_pk_bf16_f32 and the matrix
+// cores keep subnormal parts). Products and their sums then carry kScale^2, and
+// one past 2^96 overflows, which shows in the sum. The multiplication takes the
+// two instructions a pair that noticing small values would take.
+constexpr float kScale = 0x1p16f, kUnscale = 0x1p-32f;
+
 // The smallest magnitudes seen, as (2 * bf16 bits - 1) per 16-bit half: zero
 // wraps to the largest value, so it never counts. Parts of a value of at least
 // 2^-100 (kSmallest) lose nothing to bf16's smallest subnormal.

@@ -1,6 +1,6 @@
 """Products on bf16 parts (csrc/split_bf16.hpp) where the parts alone are not
-enough: values below 2^-100 (their third part meets bf16's smallest
-subnormal), infinities and NaN (an infinity minus its own first part), and the
+enough: values whose own parts would meet bf16's smallest subnormal (which
+the scale ahead of the split lifts above it), infinities and NaN (an infinity minus its own first part), and the
 top of the FP32 range (the partial products overflow one by one). The kernels
 must notice each and give what FP32 arithmetic gives.
 
@@ -55,6 +55,18 @@ def check(got, a, b, k):
     assert (np.abs(got[finite].astype(np.float64) - want[finite]) <= bound).all()
 
 
+def product(runtime, m, n, k, a, b):
+    kernel = runtime.compile({"op": "gemm", "m": m, "n": n, "k": k, "tiled": True})
+    assert kernel.launch["kernel"] == "gemm_f32_ring_128x128x32"
+    bufs = [runtime.resident(a), runtime.resident(b), runtime.alloc(m * n)]
+    print(f"ring {m}x{n}x{k}", flush=True)
+    runtime.execute([(kernel, bufs)], 1)
+    got = runtime.download(bufs[2]).reshape(m, n)
+    for x in bufs:
+        x.free()
+    return got
+
+
 @pytest.mark.parametrize("name", CASES)
 @pytest.mark.parametrize("m,n,k", [(2048, 2048, 512), (2560, 2560, 1024)])  # one tile a workgroup; runs of one and two
 def test_persistent_gemm_special_values(runtime, name, m, n, k):
@@ -87,6 +99,67 @@ def test_persistent_gate_up_special_values(runtime, name):
         t.free()
     check(got_g, a, b, k)
     check(got_u, a, np.ascontiguousarray(b[:, ::-1]), k)
+
+
+@pytest.mark.parametrize("side", ["a", "b"])
+@pytest.mark.parametrize("m,n,k", [(2048, 2048, 512), (2560, 2560, 1024)])
+def test_persistent_gemm_keeps_subnormals(runtime, side, m, n, k):
+    # Every nonzero of one operand lies below 2^-134, where bf16 holds nothing.
+    tiny = (orc.values(m * k if side == "a" else k * n, 0x73, 1.0).astype(np.float64) * 2.0 ** -134).astype(np.float32)
+    other = orc.values(k * n if side == "a" else m * k, 0x74, 1.0) * np.float32(1e30)
+    a, b = (tiny, other) if side == "a" else (other, tiny)
+    got = product(runtime, m, n, k, a, b)
+    assert np.abs(got).max() > 1e-11
+    check(got, a.reshape(m, k), b.reshape(k, n), k)
+
+
+def test_persistent_gemm_small_products(runtime):
+    # Products near the smallest normals: products of their parts lie below them.
+    m, n, k = 2048, 2048, 512
+    a, b = orc.values(m * k, 0x75, 1.0) * np.float32(2.0 ** -55), orc.values(k * n, 0x76, 1.0) * np.float32(2.0 ** -55)
+    check(product(runtime, m, n, k, a, b), a.reshape(m, k), b.reshape(k, n), k)
+
+
+@pytest.mark.parametrize("special", [1e-35, 1e-41])
+def test_persistent_gemm_special_value_stays_in_its_row_and_column(runtime, special):
+    # How an output is computed depends on its own row and column alone, so one
+    # tiny, infinite or huge operand leaves all other outputs' bits (and so
+    # the work done for them) as they were.
+    m, n, k = 2560, 2560, 512  # two tiles in some workgroups
+    a, b = orc.values(m * k, 0x77, 1.0).reshape(m, k), orc.values(k * n, 0x78, 1.0).reshape(k, n)
+    plain = product(runtime, m, n, k, a, b)
+    a[5, 3] = b[k // 2, 700] = special
+    got = product(runtime, m, n, k, a, b)
+    plain[5], plain[:, 700] = got[5], got[:, 700]
+    np.testing.assert_array_equal(got, plain)
+    check(got, a, b, k)
+
+
+@pytest.mark.parametrize("special", [1e-35, 1e-41])
+@pytest.mark.parametrize("where", ["x", "gate", "up"])
+def test_persistent_gate_up_bits_with_a_special_value(runtime, special, where):
+    # A special value in one operand: the fused launch's bits stay those of
+    # each product launched alone.
+    m, n, k = 2048, 2048, 512  # two tiles of 128x64 a workgroup fused, one of 128x128 alone
+    data = {"x": orc.values(m * k, 0x79, 1.0), "gate": orc.values(k * n, 0x7A, 1.0), "up": orc.values(k * n, 0x7B, 1.0)}
+    data[where][(m * k if where == "x" else k * n) // 2 + 77] = special
+    gemm = runtime.compile({"op": "gemm", "m": m, "n": n, "k": k, "tiled": True})
+    assert gemm.launch["kernel"] == "gemm_f32_ring_128x128x32"
+    swiglu = runtime.compile({"op": "swi_glu", "len": m * n})
+    x, wg, wu = (runtime.resident(t) for t in data.values())
+    g, u, d = (runtime.alloc(m * n) for _ in range(3))
+    jobs = [(gemm, [x, wg, g]), (gemm, [x, wu, u]), (swiglu, [g, u, d])]
+    assert runtime.plan(jobs) == [("gate_up_swiglu", 0)]
+    print(f"dual ring {special} in {where}", flush=True)
+    runtime.execute(jobs, 1)
+    fused = [runtime.download(t) for t in (g, u, d)]
+    for job in jobs:
+        runtime.execute([job], 1)
+    alone = [runtime.download(t) for t in (g, u, d)]
+    for t in (x, wg, wu, g, u, d):
+        t.free()
+    for f, w, name in zip(fused, alone, ("gate", "up", "act")):
+        np.testing.assert_array_equal(f, w, err_msg=name)
 
 
 def attend(runtime, heads, seq, dim, causal, q, k, v):
