@@ -53,8 +53,11 @@ namespace {
 // scaled back before they are stored. An infinity minus its own first part is
 // NaN, and scaled values past 2^112 and sums past 2^96 overflow: a wave whose
 // sums are not all finite computes its outputs again from global memory with
-// FP32 MFMAs, so infinities, NaN and overflow come out as FP32 arithmetic
-// gives them, at about a tenth of the speed.
+// FP32 MFMAs and takes those in the place of the sums that are not, so
+// infinities, NaN and overflow come out as FP32 arithmetic gives them, at about
+// a tenth of the speed. Which way an output is computed thus depends on its own
+// row and column alone, not on its tile's other outputs: every form of this
+// kernel gives it the same bits.
 //
 // Requires M, N multiples of 128 (N of 64 for DUAL), K a multiple of 256,
 // 16-byte aligned operands, 32-bit load offsets inside a tile.
@@ -360,15 +363,14 @@ __global__ __launch_bounds__(ring::kThreads) __attribute__((amdgpu_waves_per_eu(
         }
     };
 
-    // The wave's outputs of the tile at (m0, n0) again, in FP32 from global
-    // memory: lane (h, c) takes k 4h on of every eight, for A row c and B
-    // columns 2c, 2c + 1 (DUAL: column c of each product).
+    // The wave's outputs of the tile at (m0, n0) that are not finite, again in
+    // FP32 from global memory: lane (h, c) takes k 4h on of every eight, for A
+    // row c and B columns 2c, 2c + 1 (DUAL: column c of each product).
     auto again = [&](int m0, int n0) __attribute__((always_inline)) {
         const float *a = A + size_t(m0 + 32 * wm + c) * size_t(K) + 4 * h;
         const size_t col = size_t(4 * h) * size_t(N) + n0 + (DUAL ? 32 * wn + c : 64 * wn + 2 * c);
         const float *b0 = B + col, *b1 = DUAL ? B2 + col : B + col + 1;
-        f32x16 run[2] = {};
-        acc[0] = acc[1] = f32x16{};
+        f32x16 run[2] = {}, whole[2] = {};
         for (int k = 0; k < K; k += 8) {
             const f32x4 x = *reinterpret_cast<const f32x4 *>(a + k);
 #pragma unroll
@@ -380,11 +382,16 @@ __global__ __launch_bounds__(ring::kThreads) __attribute__((amdgpu_waves_per_eu(
             if ((k & 127) == 120) {
 #pragma unroll
                 for (int j = 0; j < 2; ++j) {
-                    acc[j] += run[j];
+                    whole[j] += run[j];
                     run[j] = f32x16{};
                 }
             }
         }
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+                if (acc[j][v] * 0.f != 0.f) acc[j][v] = whole[j][v];
     };
 
     for (int t = 0; t < mine; ++t) {

@@ -120,7 +120,7 @@ def test_persistent_gemm_small_products(runtime):
     check(product(runtime, m, n, k, a, b), a.reshape(m, k), b.reshape(k, n), k)
 
 
-@pytest.mark.parametrize("special", [1e-35, 1e-41])
+@pytest.mark.parametrize("special", [1e-35, 1e-41, np.inf, 3e38])
 def test_persistent_gemm_special_value_stays_in_its_row_and_column(runtime, special):
     # How an output is computed depends on its own row and column alone, so one
     # tiny, infinite or huge operand leaves all other outputs' bits (and so
@@ -135,7 +135,7 @@ def test_persistent_gemm_special_value_stays_in_its_row_and_column(runtime, spec
     check(got, a, b, k)
 
 
-@pytest.mark.parametrize("special", [1e-35, 1e-41])
+@pytest.mark.parametrize("special", [1e-35, 1e-41, np.inf, np.nan, 3e38])
 @pytest.mark.parametrize("where", ["x", "gate", "up"])
 def test_persistent_gate_up_bits_with_a_special_value(runtime, special, where):
     # A special value in one operand: the fused launch's bits stay those of
