@@ -22,12 +22,13 @@
 // (2-norm, relative): 4.1e-7 where that kernel had 5.4e-7 (H128 S4096 D128
 // causal), 6.3e-7 for 7.8e-7 (H24 S1531 D80).
 //
-// What the parts do not carry (split_bf16.hpp) is noticed and done again from
-// global memory with FP32 MFMAs, per wave: non-finite sums (infinities, NaN or
-// overflow among the operands), queries outside [2^-64, 2^64] in log2 units,
-// and, for the whole block, a value of V below 2^-100. With such queries out of
-// the way a tiny K moves no score by more than 2^-70. Weights below 2^-100 of
-// the reference weight keep fewer than 24 bits.
+// V is scaled before it is split and the outputs are scaled back, so every
+// finite V is carried exactly (split_bf16.hpp). What the parts do not carry is
+// noticed and done again from global memory with FP32 MFMAs, per wave:
+// non-finite sums (infinities, NaN or overflow among the operands) and queries
+// outside [2^-64, 2^64] in log2 units. With such queries out of the way a tiny
+// K moves no score by more than 2^-70. Weights below 2^-100 of the reference
+// weight keep fewer than 24 bits.
 #include <type_traits>
 #include <utility>
 
@@ -209,7 +210,6 @@ attention_flash(const float *__restrict__ Q, const float *__restrict__ K, const 
     constexpr int kPairsV = VROWS / 2;
     uint32_t kparts[CH][kParts][4], vparts[2][kParts][kPairsV];
     f32x2 rest;
-    u16x2 smallest = {0xffff, 0xffff};
     auto piece_of = [&](uint32_t &out, int piece, f32x2 x) {
         const f32x2 from = piece == 0 ? x : rest;
         out = pack(from.x, from.y);
@@ -221,8 +221,7 @@ attention_flash(const float *__restrict__ Q, const float *__restrict__ K, const 
     };
     auto convert_v = [&](int j, int u, int piece) {
         const f32x2 k0 = vraw[2 * u], k1 = vraw[2 * u + 1];
-        piece_of(vparts[j][piece][u], piece, j ? f32x2{k0.y, k1.y} : f32x2{k0.x, k1.x});
-        if (piece == 2) smallest = __builtin_elementwise_min(smallest, doubled_less_one(vparts[j][0][u]));
+        piece_of(vparts[j][piece][u], piece, (j ? f32x2{k0.y, k1.y} : f32x2{k0.x, k1.x}) * kScaleV);
     };
     auto write_k = [&](int i, int p, uint32_t buf) {
         *reinterpret_cast<u32x4 *>(lds + (kwrite[i] + buf * S::kTileK) + uint32_t(p) * S::kPartK) =
@@ -596,13 +595,9 @@ attention_flash(const float *__restrict__ Q, const float *__restrict__ K, const 
     for (int b = 0; b < NB; ++b)
 #pragma unroll
         for (int v = 0; v < 16; ++v) total += acc[b][v] * 0.f;
-    volatile int *tiny = reinterpret_cast<volatile int *>(lds);
-    publish();
-    if (tid == 0) *tiny = 0;
-    publish();
-    if (__any(lossy(smallest)) && lane == 0) *tiny = 1;
-    publish();
-    if (rows && (*tiny || __any(odd_q || total != 0.f))) {
+    float unscale = kUnscaleV;
+    if (rows && __any(odd_q || total != 0.f)) {
+        unscale = 1.f;
         row_max = -INFINITY;
         row_sum = 0.f;
 #pragma unroll
@@ -657,7 +652,7 @@ attention_flash(const float *__restrict__ Q, const float *__restrict__ K, const 
 
     row_sum = halves_sum(row_sum);
     if (qi < seq) {
-        const float inv = 1.0f / row_sum;
+        const float inv = unscale / row_sum;
         float *orow = O + base + size_t(qi) * dim;
         // LDS row r of V is dim 2r (r < DP / 2) or 2 (r - DP / 2) + 1, and a
         // lane holds rows 32b + 8 (v >> 2) + 4h + (v & 3): r, r + 1 and their

@@ -66,17 +66,10 @@ __device__ inline f32x2 rest_of(f32x2 x, uint32_t p) {
 // one past 2^96 overflows, which shows in the sum. The multiplication takes the
 // two instructions a pair that noticing small values would take.
 constexpr float kScale = 0x1p16f, kUnscale = 0x1p-32f;
-
-// The smallest magnitudes seen, as (2 * bf16 bits - 1) per 16-bit half: zero
-// wraps to the largest value, so it never counts. Parts of a value of at least
-// 2^-100 (kSmallest) lose nothing to bf16's smallest subnormal.
-constexpr uint16_t kSmallest = uint16_t(2 * ((127 - 100) << 7) - 1);
-__device__ inline u16x2 doubled_less_one(uint32_t p) {
-    return __builtin_bit_cast(u16x2, p) * u16x2{2, 2} + u16x2{0xffff, 0xffff};
-}
-__device__ inline bool lossy(u16x2 smallest) {
-    return smallest.x < kSmallest || smallest.y < kSmallest;
-}
+// Attention's V meets weights that are not scaled. 2^24 keeps V's parts
+// normal numbers, which v_dot2_f32_bf16 (rest_of) needs; sums past 2^104
+// overflow.
+constexpr float kScaleV = 0x1p24f, kUnscaleV = 0x1p-24f;
 
 }  // namespace split
 }  // namespace

@@ -242,3 +242,30 @@ def test_flash_on_parts_non_finite(runtime, heads, seq, dim, causal):
     assert np.isnan(got[3, key]).all()
     rest = [r for r in range(seq) if r != key]
     assert orc.compare(got[3, rest].ravel(), want[3, rest].ravel(), 1e-5, 1e-5).status == 0
+
+
+@pytest.mark.parametrize("heads,seq,dim,causal", FLASH)
+def test_flash_on_parts_subnormal_values(runtime, heads, seq, dim, causal):
+    # Every V below 2^-134, where bf16 holds nothing; outputs keep FP32's
+    # absolute 2^-149 (and the sum of the weights its rounding).
+    n = heads * seq * dim
+    q, k = orc.normal(n, 0xB1), orc.normal(n, 0xB2)
+    v = (orc.values(n, 0xB3, 1.0).astype(np.float64) * 2.0 ** -134).astype(np.float32)
+    got, _ = attend(runtime, heads, seq, dim, causal, q, k, v)
+    want = np.asarray(orc.attention_reference(heads, seq, dim, causal, q, k, v * np.float32(2.0 ** 64)), np.float64)
+    assert np.abs(got.astype(np.float64) * 2.0 ** 64 - want).max() <= 4 * 2.0 ** -85
+
+
+@pytest.mark.parametrize("heads,seq,dim,causal", FLASH)
+@pytest.mark.parametrize("special", [1e-35, 1e-41])
+def test_flash_on_parts_tiny_value_costs_nothing(runtime, heads, seq, dim, causal, special):
+    # One tiny V in place of a zero: the other dims' bits (and so the work done
+    # for them) stay as they were.
+    n = heads * seq * dim
+    q, k, v = (orc.normal(n, s).reshape(heads, seq, dim).copy() for s in (0xB4, 0xB5, 0xB6))
+    v[:, seq // 2, 3] = 0
+    plain, _ = attend(runtime, heads, seq, dim, causal, q.ravel(), k.ravel(), v.ravel())
+    v[:, seq // 2, 3] = special
+    got, _ = attend(runtime, heads, seq, dim, causal, q.ravel(), k.ravel(), v.ravel())
+    other = [d for d in range(dim) if d != 3]
+    np.testing.assert_array_equal(got.reshape(n // dim, dim)[:, other], plain.reshape(n // dim, dim)[:, other])
