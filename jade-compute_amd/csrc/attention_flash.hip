@@ -22,13 +22,13 @@
 // (2-norm, relative): 4.1e-7 where that kernel had 5.4e-7 (H128 S4096 D128
 // causal), 6.3e-7 for 7.8e-7 (H24 S1531 D80).
 //
-// V is scaled before it is split and the outputs are scaled back, so every
-// finite V is carried exactly (split_bf16.hpp). What the parts do not carry is
-// noticed and done again from global memory with FP32 MFMAs, per wave:
-// non-finite sums (infinities, NaN or overflow among the operands) and queries
-// outside [2^-64, 2^64] in log2 units. With such queries out of the way a tiny
-// K moves no score by more than 2^-70. Weights below 2^-100 of the reference
-// weight keep fewer than 24 bits.
+// V is scaled before it is split and the outputs are scaled back, Q is scaled
+// up and K down, so every finite V and Q is carried exactly (split_bf16.hpp).
+// What the parts do not carry is noticed and done again from global memory
+// with FP32 MFMAs, per wave: non-finite sums (infinities, NaN or overflow among
+// the operands) and queries past 2^64 in log2 units. With such queries out of
+// the way the bits that a K below 2^-78 loses move no score by more than
+// 2^-38 a dim. Weights below 2^-100 of the reference weight keep fewer than 24 bits.
 #include <type_traits>
 #include <utility>
 
@@ -50,9 +50,9 @@ constexpr int kKeys = 32;      // keys per tile
 constexpr float kLazyMax = 8.0f;
 constexpr uint32_t kRawBuffer = 0x00020000;   // buffer descriptor word 3: raw buffer, 32-bit data format
 constexpr uint32_t kDeadOffset = 0x80000000u;  // past every head of at most 2 GiB: reads zero
-// Q outside this range (zero apart) takes the FP32 path: then no product of a
-// part of Q with a part of a tiny K loses more than an FP32 score's rounding.
-constexpr float kLeastQ = 0x1p-64f, kMostQ = 0x1p64f;
+// Scaled Q past this takes the FP32 path: then no product of a part of Q with a
+// part of a tiny K loses more than an FP32 score's rounding.
+constexpr float kMostQ = 0x1p64f * kScaleQ;
 
 __device__ inline float halves_max(float x) {
     const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
@@ -143,9 +143,8 @@ attention_flash(const float *__restrict__ Q, const float *__restrict__ K, const 
             if (qi < seq && d < dim) q = *reinterpret_cast<const f32x4 *>(Q + base + size_t(qi) * dim + d);
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
-                f32x2 r = {q[2 * u] * qscale, q[2 * u + 1] * qscale};
-                odd_q = odd_q || (r.x != 0.f && !(fabsf(r.x) >= kLeastQ && fabsf(r.x) <= kMostQ)) ||
-                        (r.y != 0.f && !(fabsf(r.y) >= kLeastQ && fabsf(r.y) <= kMostQ));
+                f32x2 r = f32x2{q[2 * u], q[2 * u + 1]} * (qscale * kScaleQ);
+                odd_q = odd_q || !(fabsf(r.x) <= kMostQ && fabsf(r.y) <= kMostQ);
 #pragma unroll
                 for (int w = 0; w < kParts; ++w) {
                     const uint32_t k = pack(r.x, r.y);
@@ -217,7 +216,7 @@ attention_flash(const float *__restrict__ Q, const float *__restrict__ K, const 
     };
     auto convert_k = [&](int i, int u, int piece) {
         const f32x4 k = kraw[i][u >> 1];
-        piece_of(kparts[i][piece][u], piece, u & 1 ? f32x2{k.z, k.w} : f32x2{k.x, k.y});
+        piece_of(kparts[i][piece][u], piece, (u & 1 ? f32x2{k.z, k.w} : f32x2{k.x, k.y}) * kScaleK);
     };
     auto convert_v = [&](int j, int u, int piece) {
         const f32x2 k0 = vraw[2 * u], k1 = vraw[2 * u + 1];

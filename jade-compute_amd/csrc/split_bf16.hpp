@@ -68,8 +68,9 @@ __device__ inline f32x2 rest_of(f32x2 x, uint32_t p) {
 constexpr float kScale = 0x1p16f, kUnscale = 0x1p-32f;
 // Attention's V meets weights that are not scaled. 2^24 keeps V's parts
 // normal numbers, which v_dot2_f32_bf16 (rest_of) needs; sums past 2^104
-// overflow.
-constexpr float kScaleV = 0x1p24f, kUnscaleV = 0x1p-24f;
+// overflow. Its Q is scaled up by as much and its K down, so the scores are as
+// they are without.
+constexpr float kScaleV = 0x1p24f, kUnscaleV = 0x1p-24f, kScaleQ = 0x1p24f, kScaleK = 0x1p-24f;
 
 }  // namespace split
 }  // namespace

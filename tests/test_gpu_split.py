@@ -269,3 +269,32 @@ def test_flash_on_parts_tiny_value_costs_nothing(runtime, heads, seq, dim, causa
     got, _ = attend(runtime, heads, seq, dim, causal, q.ravel(), k.ravel(), v.ravel())
     other = [d for d in range(dim) if d != 3]
     np.testing.assert_array_equal(got.reshape(n // dim, dim)[:, other], plain.reshape(n // dim, dim)[:, other])
+
+
+@pytest.mark.parametrize("heads,seq,dim,causal", FLASH)
+@pytest.mark.parametrize("special", [1e-25, 1e-42])
+def test_flash_on_parts_tiny_query_costs_nothing(runtime, heads, seq, dim, causal, special):
+    # One tiny Q element in place of a zero moves no score, so all bits (and so
+    # the work done) stay as they were.
+    n = heads * seq * dim
+    q, k, v = (orc.normal(n, s).reshape(heads, seq, dim).copy() for s in (0xB7, 0xB8, 0xB9))
+    q[:, ::20, 3] = 0
+    plain, _ = attend(runtime, heads, seq, dim, causal, q.ravel(), k.ravel(), v.ravel())
+    q[:, ::20, 3] = special
+    got, _ = attend(runtime, heads, seq, dim, causal, q.ravel(), k.ravel(), v.ravel())
+    np.testing.assert_array_equal(got, plain)
+
+
+@pytest.mark.parametrize("heads,seq,dim,causal", FLASH)
+def test_flash_on_parts_subnormal_operands(runtime, heads, seq, dim, causal):
+    # Q (or K) below 2^-110, subnormals among it, against K (or Q) as large: ordinary scores.
+    n = heads * seq * dim
+    v = orc.normal(n, 0xBC)
+    for tiny_q in (True, False):
+        small = (orc.normal(n, 0xBA).astype(np.float64) * 2.0 ** -126).astype(np.float32)
+        large = orc.normal(n, 0xBB) * np.float32(2.0 ** 124)
+        q, k = (small, large) if tiny_q else (large, small)
+        got, _ = attend(runtime, heads, seq, dim, causal, q, k, v)
+        s = (np.float32(2.0 ** 64), np.float32(2.0 ** -64))
+        want = orc.attention_reference(heads, seq, dim, causal, *((q * s[0], k * s[1]) if tiny_q else (q * s[1], k * s[0])), v)
+        assert orc.compare(got, want, 2e-5, 2e-5).status == 0, tiny_q
