@@ -2386,7 +2386,7 @@ LaunchShape gemm_f32_shape(uint32_t m, uint32_t n, uint32_t k) {
 
 bool gemm_f32_pairable(uint32_t m, uint32_t n, uint32_t k) {
     const Route r = route_for(m, n, k);
-    return r.launchable && !r.plan.big && !r.plan.ring && !r.plan.rows16 && !r.plan.direct && r.kg == 1 && r.plan.slices == 1;
+    return r.launchable && !r.plan.big && !r.plan.ring && !r.plan.direct && r.kg == 1 && r.plan.slices == 1;
 }
 
 hipError_t gemm_f32_pair(hipStream_t stream, const float *a0, const float *b0, float *c0, const float *a1,
@@ -2394,6 +2394,7 @@ hipError_t gemm_f32_pair(hipStream_t stream, const float *a0, const float *b0, f
     if (!gemm_f32_pairable(m, n, k)) return hipErrorInvalidValue;
     if (!aligned16(a0) || !aligned16(b0) || !aligned16(a1) || !aligned16(b1)) return hipErrorInvalidValue;
     const Route r = route_for(m, n, k);
+    if (r.plan.rows16) return launch_gemm_rows16_pair(stream, r.plan.rows16, a0, b0, c0, a1, b1, c1, m, n, k);
     const PairArgs pair{a1, b1, c1, r.plan.tiles_m * r.plan.tiles_n, nullptr, nullptr};
     return launch_route_tiles(stream, r, a0, b0, c0, m, n, k, pair);
 }

@@ -28,14 +28,22 @@ constexpr uint32_t kRawBuffer = 0x00020000;  // buffer descriptor word 3: raw bu
 constexpr int kSliceK = 32, kCols = 32, kRows = 16, kSlices = 2;
 
 // sum != nullptr: also sum = C + residual (both [M, N]), the stream kernel's
-// FP32 add.
+// FP32 add. Workgroups with blockIdx.y == 1 compute C1 = A1 B1 instead, an
+// independent product of the same shape.
 template <int G>
 __global__ __launch_bounds__(64 * G) void gemm_f32_rows16(const float *__restrict__ A, const float *__restrict__ B,
                                                           float *__restrict__ C, int M, int N, int K,
-                                                          const float *__restrict__ residual, float *__restrict__ sum) {
+                                                          const float *__restrict__ residual, float *__restrict__ sum,
+                                                          const float *__restrict__ A1, const float *__restrict__ B1,
+                                                          float *__restrict__ C1) {
     __shared__ float sums[G][kRows][kCols];
     const int lane = int(threadIdx.x) & 63, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
     const int g = lane >> 4, i = lane & 15, n0 = int(blockIdx.x) * kCols;
+    if (blockIdx.y == 1) {
+        A = A1;
+        B = B1;
+        C = C1;
+    }
     // Rows of A past M and rows of B past K lie past the buffers and read
     // zero; a run of A past K reads the next row and is zeroed below.
     const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
@@ -86,17 +94,34 @@ __global__ __launch_bounds__(64 * G) void gemm_f32_rows16(const float *__restric
 
 }  // namespace
 
-hipError_t launch_gemm_rows16(hipStream_t stream, int waves, const float *a, const float *b, float *c, uint32_t m,
-                              uint32_t n, uint32_t k, const float *residual, float *sum) {
+namespace {
+
+hipError_t launch(hipStream_t stream, int waves, unsigned products, const float *a, const float *b, float *c,
+                  uint32_t m, uint32_t n, uint32_t k, const float *residual, float *sum, const float *a1,
+                  const float *b1, float *c1) {
     if (m > uint32_t(kRows) || k > uint32_t(kSlices * kSliceK * waves)) return hipErrorInvalidValue;
-    const dim3 grid((n + kCols - 1) / kCols), block(64 * waves);
+    const dim3 grid((n + kCols - 1) / kCols, products), block(64 * waves);
     if (waves == 4)
-        hipLaunchKernelGGL(gemm_f32_rows16<4>, grid, block, 0, stream, a, b, c, int(m), int(n), int(k), residual, sum);
+        hipLaunchKernelGGL(gemm_f32_rows16<4>, grid, block, 0, stream, a, b, c, int(m), int(n), int(k), residual, sum,
+                           a1, b1, c1);
     else if (waves == 8)
-        hipLaunchKernelGGL(gemm_f32_rows16<8>, grid, block, 0, stream, a, b, c, int(m), int(n), int(k), residual, sum);
+        hipLaunchKernelGGL(gemm_f32_rows16<8>, grid, block, 0, stream, a, b, c, int(m), int(n), int(k), residual, sum,
+                           a1, b1, c1);
     else
         return hipErrorInvalidValue;
     return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_gemm_rows16(hipStream_t stream, int waves, const float *a, const float *b, float *c, uint32_t m,
+                              uint32_t n, uint32_t k, const float *residual, float *sum) {
+    return launch(stream, waves, 1, a, b, c, m, n, k, residual, sum, nullptr, nullptr, nullptr);
+}
+
+hipError_t launch_gemm_rows16_pair(hipStream_t stream, int waves, const float *a0, const float *b0, float *c0,
+                                   const float *a1, const float *b1, float *c1, uint32_t m, uint32_t n, uint32_t k) {
+    return launch(stream, waves, 2, a0, b0, c0, m, n, k, nullptr, nullptr, a1, b1, c1);
 }
 
 }  // namespace hipk

@@ -42,3 +42,24 @@ def test_rows16_shapes(runtime, m, n, k, waves):
         if special:
             assert np.isnan(got[:, 0]).all() and not np.isfinite(got[m - 1]).any()
         np.testing.assert_array_equal(total[rows, cols], got[rows, cols] + x.reshape(m, n)[rows, cols])
+
+
+@pytest.mark.parametrize("m,n,k", [(8, 256, 128), (16, 33, 31), (3, 31, 48), (7, 100, 257)])
+def test_rows16_pairs(runtime, m, n, k):
+    # Two products of one shape run as one launch, each output bit for bit its own launch's.
+    gemm = runtime.compile({"op": "gemm", "m": m, "n": n, "k": k, "tiled": True})
+    assert gemm.launch["kernel"].startswith("gemm_f32_rows16"), gemm.launch
+    x, wg, wu = (runtime.resident(orc.values(c, s, 1.0)) for c, s in ((m * k, 0x64), (k * n, 0x65), (k * n, 0x66)))
+    c = [runtime.alloc(m * n) for _ in range(2)]
+    jobs = [(gemm, [x, wg, c[0]]), (gemm, [x, wu, c[1]])]
+    assert runtime.plan(jobs) == [("pair", 0)]
+    print(f"rows16 pair {m}x{n}x{k}", flush=True)
+    runtime.execute(jobs, 2)
+    both = [runtime.download(t) for t in c]
+    for job in jobs:
+        runtime.execute([job], 1)
+    alone = [runtime.download(t) for t in c]
+    for t in (x, wg, wu, *c):
+        t.free()
+    for got, want in zip(both, alone):
+        np.testing.assert_array_equal(got, want)
