@@ -164,8 +164,7 @@ def measure(workloads, steps, warmup, min_repeats=SAMPLE_REPEATS):
 
 def on_parts(launch_kernel):
     """Whether a launch runs its products on the bf16 matrix cores."""
-    return launch_kernel.startswith("gemm_f32_ring") or (
-        launch_kernel.startswith("attention_online_mfma_d") and not launch_kernel.endswith("_split"))
+    return launch_kernel.startswith(("gemm_f32_ring", "attention_flash"))
 
 
 def peak_of(launch_kernel):
@@ -175,10 +174,10 @@ def peak_of(launch_kernel):
 def symbol_of(launch_kernel):
     """The kernel symbol prefix (as rocprofv3 names it) of a launch that
     jr_kernel_describe reports as `launch_kernel`."""
-    if launch_kernel.startswith("attention") and on_parts(launch_kernel):
-        return "attention_flash"
-    for prefix in ("gemm_f32_ring", "gemm_f32_mfma_256", "gemm_f32_direct", "gemm_f32_dual_swiglu",
-                   "attention_online_mfma", "attention_pairs_mfma"):
+    if launch_kernel.startswith("attention_online_mfma16"):
+        return "attention_pairs_mfma"
+    for prefix in ("gemm_f32_ring", "gemm_f32_rows16", "gemm_f32_mfma_256", "gemm_f32_direct", "gemm_f32_dual_swiglu",
+                   "attention_flash", "attention_online_mfma"):
         if launch_kernel.startswith(prefix):
             return prefix
     return "gemm_f32_mfma"
@@ -356,7 +355,7 @@ def bench_mlp(rt, batch, width, hidden, steps, warmup):
             ms = t["ms_per_step"]
             spec = dict(specs)[name]
             per[name] = {"ms": ms, "tflops": gemm_flops[name] / (ms * 1e-3) / 1e12,
-                         "frac_mfma": gemm_flops[name] / (ms * 1e-3) / 1e12 / PEAK_FP32_MFMA_TFLOPS,
+                         "frac_mfma": gemm_flops[name] / (ms * 1e-3) / 1e12 / peak_of(job[0].launch["kernel"]),
                          "kernel": job[0].launch["kernel"], "shape": f"{spec['m']}x{spec['n']}x{spec['k']}"}
     total_flops = sum(gemm_flops.values())
     for buf in (xg, ng, wgg, wug, wdg, normalized, gate, up, act, proj, out):
@@ -926,7 +925,7 @@ def main():
         for causal in (False, True):
             r = bench_attention(rt, 8, 1024, 64, causal, K, W)
             c3["causal" if causal else "noncausal"] = {
-                "ms": r["ms_per_step"], "tflops": r["tflops"], "frac_mfma": r["tflops"] / PEAK_FP32_MFMA_TFLOPS,
+                "ms": r["ms_per_step"], "tflops": r["tflops"], "frac_mfma": r["tflops"] / peak_of(r["kernel"]),
                 "min_ms": r["min_ms_per_step"], "max_ms": r["max_ms_per_step"], "kernel": r["kernel"]}
         extra["attention_c3_b1h8s1024d64"] = c3
         log(f"  C3 {c3['noncausal']['tflops']:.1f} / {c3['causal']['tflops']:.1f} TFLOP/s")
@@ -964,7 +963,7 @@ def main():
                         (4096, 11008, 4096)):
             r = bench_gemm(rt, m, n, k, K, W)
             sweep[f"{m}x{n}x{k}"] = {"ms": r["ms_per_step"], "tflops": r["tflops"],
-                                     "frac_mfma": r["tflops"] / PEAK_FP32_MFMA_TFLOPS,
+                                     "frac_mfma": r["tflops"] / peak_of(r["kernel"]),
                                      "min_ms": r["min_ms_per_step"], "max_ms": r["max_ms_per_step"],
                                      "kernel": r["kernel"]}
             log(f"  sweep {m}x{n}x{k} {r['tflops']:.1f} TFLOP/s")

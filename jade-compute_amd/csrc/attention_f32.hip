@@ -1455,12 +1455,15 @@ LaunchShape attention_online_shape(uint32_t heads, uint32_t seq, uint32_t dim, b
     const uint32_t bq = 32u * nw;
     const SplitPlan plan = split_plan(heads, seq, causal);
     const uint32_t splits = plan.slices;
-    const uint32_t lds = splits <= 1 && on_parts(seq, dim) ? attention_flash_lds_bytes(dim, nw)
+    const bool flash = splits <= 1 && on_parts(seq, dim);
+    const uint32_t lds = flash ? attention_flash_lds_bytes(dim, nw)
                          : dp == 32 ? lds_bytes<32>(nw) : dp == 64 ? lds_bytes<64>(nw) : lds_bytes<128>(nw);
+    static const char *const flash_names[4] = {"attention_flash_d32", "attention_flash_d64", "attention_flash_d96",
+                                               "attention_flash_d128"};
     static const char *const names[2][3] = {
         {"attention_online_mfma_d32", "attention_online_mfma_d64", "attention_online_mfma_d128"},
         {"attention_online_mfma_d32_split", "attention_online_mfma_d64_split", "attention_online_mfma_d128_split"}};
-    return {names[splits > 1][dp == 32 ? 0 : dp == 64 ? 1 : 2],
+    return {flash ? flash_names[(dim - 1) / 32] : names[splits > 1][dp == 32 ? 0 : dp == 64 ? 1 : 2],
             {splits > 1 ? plan.live : heads, splits > 1 ? 1u : (seq + bq - 1) / bq, 1},
             {uint32_t(nw) * 64u, 1, 1},
             lds};

@@ -194,3 +194,14 @@ def test_short_workloads_sample_at_least_a_millisecond(bench, monkeypatch):
     rt = FakeRuntime()
     out = bench.measure({"w": bench.Workload(rt, [], 1)}, 50, 0)
     assert out["w"]["sample_steps"] == [10] * bench.SAMPLES
+
+
+@pytest.mark.parametrize("launch,symbol,parts", [
+    ("gemm_f32_ring_128x128x32", "gemm_f32_ring", True), ("attention_flash_d128", "attention_flash", True),
+    ("attention_online_mfma_d128", "attention_online_mfma", False),  # head dims without 16-byte rows
+    ("attention_online_mfma_d64_split", "attention_online_mfma", False),
+    ("attention_online_mfma16_d64_pairs", "attention_pairs_mfma", False),
+    ("gemm_f32_rows16_w4", "gemm_f32_rows16", False), ("gemm_f32_mfma_64x64x32_k4", "gemm_f32_mfma", False)])
+def test_launch_names_their_kernel_and_peak(bench, launch, symbol, parts):
+    assert bench.symbol_of(launch) == symbol
+    assert bench.peak_of(launch) == (bench.PEAK_PARTS_TFLOPS if parts else bench.PEAK_FP32_MFMA_TFLOPS)

@@ -225,13 +225,13 @@ def test_random_shapes(runtime):
 
 @pytest.mark.parametrize("causal", [False, True])
 def test_unsplit_grid_padded_dims_and_ragged_tile(runtime, causal):
-    # The flash kernel's K/V buffer loads: head dim 96 runs in the 128-dim
-    # kernel (the lanes of dims 96-127 read zero from an offset past the
-    # buffer), and seq 1000 ends inside a 64-key tile (rows past seq lie past
-    # the head's buffer and read zero).
+    # The flash kernel's K/V buffer loads: head dim 96 stages 128 dims (the
+    # lanes of dims 96-127 read zero from an offset past the buffer), and seq
+    # 1000 ends inside a 32-key tile (rows past seq lie past the head's buffer
+    # and read zero).
     h, s, d = 32, 1000, 96
     kernel = runtime.compile({"op": "attention_online", "heads": h, "seq": s, "dim": d, "causal": causal})
-    assert kernel.launch["kernel"].startswith("attention_online_mfma_d128"), kernel.launch
+    assert kernel.launch["kernel"] == "attention_flash_d96", kernel.launch
     assert "split" not in kernel.launch["kernel"] and kernel.description["workspace_bytes"] == 0, kernel.launch
     n = h * s * d
     q, k, v = orc.normal(n, 0x4141), orc.normal(n, 0x4242), orc.normal(n, 0x4343)

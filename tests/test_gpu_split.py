@@ -166,6 +166,7 @@ def attend(runtime, heads, seq, dim, causal, q, k, v):
     kernel = runtime.compile({"op": "attention_online", "heads": heads, "seq": seq, "dim": dim, "causal": causal})
     print(f"attention H{heads} S{seq} D{dim} causal {causal}: {kernel.launch}", flush=True)
     bufs = [runtime.resident(x) for x in (q, k, v)] + [runtime.alloc(heads * seq * dim)]
+    assert kernel.launch["kernel"].startswith("attention_flash"), kernel.launch
     runtime.execute([(kernel, bufs)], 2)
     got = runtime.download(bufs[3])
     for x in bufs:
@@ -186,7 +187,7 @@ def test_flash_on_parts_shapes(runtime, heads, seq, dim, causal, threads):
     n = heads * seq * dim
     q, k, v = orc.normal(n, 0x81), orc.normal(n, 0x82), orc.normal(n, 0x83)
     got, launch = attend(runtime, heads, seq, dim, causal, q, k, v)
-    assert launch["block"][0] == threads and "split" not in launch["kernel"], launch
+    assert launch["block"][0] == threads and launch["kernel"] == f"attention_flash_d{(dim + 31) // 32 * 32}", launch
     want = orc.attention_reference(heads, seq, dim, causal, q, k, v)
     # FP32 rounding of scores of a few units and of sums of weights: 1e-5 of the unit-sized values.
     assert orc.compare(got, want, 1e-5, 1e-5).status == 0

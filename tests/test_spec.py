@@ -357,10 +357,16 @@ def test_noalloc_scratch_covers_every_split_plan():
 
 @pytest.mark.parametrize("heads,seq,dim,causal,kernel,blocks", [
     # Grids that fill the chip with 128-query blocks: the flash kernel.
-    (128, 4096, 128, True, "attention_online_mfma_d128", 128),
-    (64, 2048, 128, True, "attention_online_mfma_d128", 64),
-    (32, 2048, 64, True, "attention_online_mfma_d64", 32),
-    (1, 64, 64, True, "attention_online_mfma_d64", 1),
+    (128, 4096, 128, True, "attention_flash_d128", 128),
+    (64, 2048, 128, True, "attention_flash_d128", 64),
+    (32, 2048, 64, True, "attention_flash_d64", 32),
+    (1, 64, 64, True, "attention_flash_d64", 1),
+    (24, 1531, 80, False, "attention_flash_d96", 24),
+    (272, 129, 32, False, "attention_flash_d32", 272),
+    # The same without 16-byte rows: FP32 products.
+    (64, 2048, 126, True, "attention_online_mfma_d128", 64),
+    (24, 1531, 81, False, "attention_online_mfma_d128", 24),
+    (272, 129, 31, False, "attention_online_mfma_d32", 272),
     # Config C3: pairs of 16-query blocks, 256 workgroups.
     (8, 1024, 64, True, "attention_online_mfma16_d64_pairs", 256),
     (8, 1024, 64, False, "attention_online_mfma16_d64_pairs", 256),
