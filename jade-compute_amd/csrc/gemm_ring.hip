@@ -51,7 +51,7 @@ namespace {
 // The operands are scaled before they are split, so that every finite value is
 // carried exactly, subnormals among them (split_bf16.hpp), and the sums are
 // scaled back before they are stored. An infinity minus its own first part is
-// NaN, and scaled values past 2^112 and sums past 2^96 overflow: a wave whose
+// NaN, and values past 2^111 and sums past 2^96 overflow once scaled: a wave whose
 // sums are not all finite computes its outputs again from global memory with
 // FP32 MFMAs and takes those in the place of the sums that are not, so
 // infinities, NaN and overflow come out as FP32 arithmetic gives them, at about

@@ -5,8 +5,11 @@
 // apiece: 24 in all; the residuals are exact FP32 subtractions). A product of
 // two such values is the sum of nine products of parts; the six of the three
 // largest orders are taken on v_mfma_f32_32x32x16_bf16, whose products are
-// exact and whose sums are FP32, and the three left out are below 2^-26 of the
-// product, a quarter of an FP32 product's own rounding.
+// exact and whose sums are FP32. The three left out come to less than 2^-24 of
+// the product at worst (0.995 of that, over all mantissas), as much as an FP32
+// product's own rounding, and to 2^-27.5 in the root mean square, so a single
+// product can be off by an ulp where FP32's is off by half of one, and a sum
+// of many is closer than FP32 products with FP32 sums leave it.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -61,15 +64,16 @@ __device__ inline f32x2 rest_of(f32x2 x, uint32_t p) {
 
 // Operands are scaled by kScale before they are split: FP32's smallest
 // subnormal, 2^-149, becomes 2^-133, bf16's, so every finite value splits
-// exactly as long as it stays below 2^112 (v_cvt_pk_bf16_f32 and the matrix
-// cores keep subnormal parts). Products and their sums then carry kScale^2, and
-// one past 2^96 overflows, which shows in the sum. The multiplication takes the
-// two instructions a pair that noticing small values would take.
+// exactly as long as it stays below 2^111 (v_cvt_pk_bf16_f32 and the matrix
+// cores keep subnormal parts; past 2^111 a first part may round to infinity).
+// Products and their sums then carry kScale^2, and one past 2^96 overflows,
+// which shows in the sum. The multiplication takes the two instructions a pair
+// that noticing small values would take.
 constexpr float kScale = 0x1p16f, kUnscale = 0x1p-32f;
-// Attention's V meets weights that are not scaled. 2^24 keeps V's parts
-// normal numbers, which v_dot2_f32_bf16 (rest_of) needs; sums past 2^104
-// overflow. Its Q is scaled up by as much and its K down, so the scores are as
-// they are without.
+// Attention's V meets weights that are not scaled. 2^24 keeps V's parts normal
+// numbers, whatever v_dot2_f32_bf16 (rest_of) makes of subnormal ones; sums past
+// 2^103 may overflow. Its Q is scaled up by as much and its K down, so the
+// scores are as they are without.
 constexpr float kScaleV = 0x1p24f, kUnscaleV = 0x1p-24f, kScaleQ = 0x1p24f, kScaleK = 0x1p-24f;
 
 }  // namespace split

@@ -3,11 +3,51 @@
 stage fill each part's 128 rows of A and of B once; the operand reads of both
 half-stages return the k and the row or column that the MFMA layout needs; the
 reads cover every bank evenly; the buffer offsets stay inside a tile; and no
-buffer is written while a wave may still read it."""
+buffer is written while a wave may still read it. And of the split itself
+(csrc/split_bf16.hpp): exact for every finite value in range, and how much the
+three products of parts that are not taken can amount to."""
 import numpy as np
 import pytest
 
 PART, B_REGION, STAGE = 8192, 3 * 8192, 6 * 8192
+
+
+def parts_of(x):
+    """The three bf16 parts of FP32 values, each held in FP32, and what they leave."""
+    parts, rest = [], x
+    for _ in range(3):
+        bits = rest.view(np.uint32).astype(np.uint64)
+        part = ((bits + 0x7FFF + ((bits >> 16) & 1)) >> 16 << 16).astype(np.uint32).view(np.float32)
+        parts.append(part)
+        rest = rest - part
+    return parts, rest
+
+
+# The operands' scale and the largest exponent that stays in range with it: GEMM; attention's V and Q.
+@pytest.mark.parametrize("scale,top,least", [(2.0 ** 16, 110, 0.0), (2.0 ** 24, 102, 2.0 ** -126)])
+def test_split_of_scaled_values_is_exact(scale, top, least):
+    rng = np.random.default_rng(1)
+    mantissas = np.unique(np.concatenate([rng.integers(0, 1 << 23, 4096), [0, 1, 2, 0x7FFF, 0x8000, 0x8001, 0x7F7FFF,
+                                                                           0x7F8000, 0x7FFFFF]])).astype(np.uint32)
+    for exponent in range(0, 127 + top + 1):  # 0: subnormals and zero
+        x = (mantissas | np.uint32(exponent << 23)).view(np.float32)
+        parts, rest = parts_of(x * np.float32(scale))
+        assert not rest.any() and np.isfinite(parts[0]).all()
+        sizes = np.abs(np.stack(parts))
+        # No part below what the instructions on the way keep (0: bf16's subnormals).
+        assert (sizes[sizes > 0] >= least).all()
+
+
+def test_products_left_out_stay_below_half_an_ulp():
+    x = (np.arange(1 << 23, dtype=np.uint32) | np.uint32(0x3F800000)).view(np.float32)
+    (_, second, third), _ = parts_of(x)
+    p1, p2 = (np.abs(p.astype(np.float64)) / x for p in (second, third))
+    assert 2 * p1.max() * p2.max() + p2.max() ** 2 < 0.996 * 2.0 ** -24
+    rng = np.random.default_rng(2)
+    i, j = rng.integers(0, 1 << 23, (2, 1 << 20))
+    s, t, x = second.astype(np.float64), third.astype(np.float64), x.astype(np.float64)
+    lost = (s[i] * t[j] + t[i] * s[j] + t[i] * t[j]) / (x[i] * x[j])
+    assert np.sqrt((lost ** 2).mean()) < 2.0 ** -27.4
 
 
 def swz(row):
