@@ -1152,9 +1152,8 @@ __device__ inline void issue_stage(const float *__restrict__ A, const float *__r
 }
 
 // One (64 TM) x 64 tile at (m0, n0): its gate product in waves 0-3, its up
-// product in waves 4-7. FOLD: stages per run before each fold, that of the
-// kernel each product would run on alone.
-template <int TM, int FOLD>
+// product in waves 4-7.
+template <int TM>
 __device__ inline void tile(const float *__restrict__ A, const float *__restrict__ Bg, const float *__restrict__ Bu,
                             float *__restrict__ G, float *__restrict__ U, float *__restrict__ Act, int N, int K,
                             int m0, int n0, float *smem) {
@@ -1175,12 +1174,12 @@ __device__ inline void tile(const float *__restrict__ A, const float *__restrict
     issue_stage<TM>(A, B, N, K, m0, n0, 0, lds0, wave, lane);
     drain_vmem();
     __syncthreads();
-    // The LDS-direct loop's schedule: partial sums over FOLD stages, then a
-    // fold.
+    // The LDS-direct loop's schedule: partial sums over kFoldStages stages, then
+    // a fold.
     f32x16 part[TM][1];
-    for (int kt = 0; kt < nk; kt += FOLD) {
+    for (int kt = 0; kt < nk; kt += kFoldStages) {
 #pragma unroll
-        for (int uu = 0; uu < FOLD; ++uu) {
+        for (int uu = 0; uu < kFoldStages; ++uu) {
             const int k = kt + uu, u = uu & 1;
             if (k < nk) {
                 const float *cur = smem + u * S::kStage;
@@ -1200,7 +1199,7 @@ __device__ inline void tile(const float *__restrict__ A, const float *__restrict
                     mma_stage_swz<TM, 1, true>(cur, cur + Tl::kAStageS + group * Tl::kBStageS, wm, wn, lane, part, spread);
                 else
                     mma_stage_swz<TM, 1, false>(cur, cur + Tl::kAStageS + group * Tl::kBStageS, wm, wn, lane, part, spread);
-                if (uu == FOLD - 1) {
+                if (uu == kFoldStages - 1) {
 #pragma unroll
                     for (int i = 0; i < TM; ++i) acc[i][0] += part[i][0];
                 }
@@ -1210,7 +1209,7 @@ __device__ inline void tile(const float *__restrict__ A, const float *__restrict
             }
         }
     }
-    if (nk % FOLD != 0) {  // the last, shorter run
+    if (nk % kFoldStages != 0) {  // the last, shorter run
 #pragma unroll
         for (int i = 0; i < TM; ++i) acc[i][0] += part[i][0];
     }
@@ -1245,7 +1244,6 @@ __device__ inline void tile(const float *__restrict__ A, const float *__restrict
 // Workgroups [0, tiles_m body_tn) take the 128x64 tiles of columns
 // [0, 64 body_tn) in the XCD-grouped order; the rest take the 64x64 tiles of
 // the columns right of them, row-major.
-template <int FOLD>
 __global__ __launch_bounds__(dual::kThreads) void gemm_f32_dual_swiglu(
     const float *__restrict__ A, const float *__restrict__ Bg, const float *__restrict__ Bu, float *__restrict__ G,
     float *__restrict__ U, float *__restrict__ Act, int N, int K, int tiles_m, int tiles_n, int body_tn) {
@@ -1255,10 +1253,10 @@ __global__ __launch_bounds__(dual::kThreads) void gemm_f32_dual_swiglu(
         const int pos = xcd_order(int(blockIdx.x), body);
         int tm, tn;
         grouped_tile(pos, tiles_m, body_tn, tm, tn);
-        dual::tile<2, FOLD>(A, Bg, Bu, G, U, Act, N, K, tm * 128, tn * 64, smem);
+        dual::tile<2>(A, Bg, Bu, G, U, Act, N, K, tm * 128, tn * 64, smem);
     } else {
         const int pos = int(blockIdx.x) - body, edge_n = tiles_n - body_tn;
-        dual::tile<1, FOLD>(A, Bg, Bu, G, U, Act, N, K, (pos / edge_n) * 64, (body_tn + pos % edge_n) * 64, smem);
+        dual::tile<1>(A, Bg, Bu, G, U, Act, N, K, (pos / edge_n) * 64, (body_tn + pos % edge_n) * 64, smem);
     }
 }
 
@@ -2421,9 +2419,9 @@ hipError_t gemm_f32_residual(hipStream_t stream, const float *a, const float *b,
 
 bool gemm_f32_dual_swiglu_fits(uint32_t m, uint32_t n, uint32_t k) {
     // The plan each product would take alone must give the fused kernel's
-    // bits: the 128x64 tile (paired), or the persistent kernel, whose outputs
-    // take the same MFMA steps over k; the fused launch then folds as that
-    // plan does (every kFoldStages or ring::kFoldRun stages).
+    // bits: the 128x64 tile (paired), or the persistent kernel, which then runs
+    // the fused launch too (gemm_ring.hip), with the same steps over k for
+    // every output.
     const Route r = route_for(m, n, k);
     const Plan &p = r.plan;
     const bool same_bits = r.launchable && (p.ring || (gemm_f32_pairable(m, n, k) && p.tm == 2 && p.tn == 1));
@@ -2436,8 +2434,8 @@ bool gemm_f32_dual_swiglu_fits(uint32_t m, uint32_t n, uint32_t k) {
 // of at most half the CUs' worth of tiles that fills whole tile columns, those
 // columns' tiles run as twice as many 64x64 tiles, so the busiest CU holds
 // floor(tiles / CUs) + 1/2 tiles of work instead of floor(tiles / CUs) + 1.
-// The MLP's 4096x2816 outputs: 1408 tiles, 128 past five rounds, four
-// columns of 32 tiles.
+// 4096x2816 outputs (with a K that the persistent kernel does not take): 1408
+// tiles, 128 past five rounds, four columns of 32 tiles.
 int dual_edge_columns(int tiles_m, int tiles_n) {
     const int tiles = tiles_m * tiles_n, rem = tiles % kCUs;
     if (tiles <= kCUs || rem == 0 || rem > kCUs / 2 || rem % tiles_m != 0) return 0;
@@ -2449,13 +2447,13 @@ hipError_t gemm_f32_dual_swiglu(hipStream_t stream, const float *a, const float 
     if (!gemm_f32_dual_swiglu_fits(m, n, k) || !aligned16(a) || !aligned16(bg) || !aligned16(bu))
         return hipErrorInvalidValue;
     const int tiles_m = int(m / dual::T::kBM), tiles_n = int(n / dual::T::kBN);
-    const int edge_n = dual_edge_columns(tiles_m, tiles_n), body_tn = tiles_n - edge_n;
-    const unsigned grid = unsigned(tiles_m * body_tn + 2 * tiles_m * edge_n);
     if (route_for(m, n, k).plan.ring)
         return launch_gemm_ring_swiglu(stream, a, bg, bu, g, u, act, n, k, tiles_m, tiles_n,
                                        unsigned(std::min(tiles_m * tiles_n, kCUs)));
-    hipLaunchKernelGGL(gemm_f32_dual_swiglu<kFoldStages>, dim3(grid), dim3(dual::kThreads), 0, stream, a, bg,
-                           bu, g, u, act, int(n), int(k), tiles_m, tiles_n, body_tn);
+    const int edge_n = dual_edge_columns(tiles_m, tiles_n), body_tn = tiles_n - edge_n;
+    const unsigned grid = unsigned(tiles_m * body_tn + 2 * tiles_m * edge_n);
+    hipLaunchKernelGGL(gemm_f32_dual_swiglu, dim3(grid), dim3(dual::kThreads), 0, stream, a, bg, bu, g, u, act,
+                       int(n), int(k), tiles_m, tiles_n, body_tn);
     return hipGetLastError();
 }
 

@@ -44,11 +44,11 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kBK = 32;
 // Stages whose products the LDS-direct tile loops (and the fused gate/up
-// kernel where it stands in for them, which must match them bit for bit) sum
-// in MFMA accumulators before each fold into the running sums: 4 stages,
-// 128 k. Eight measured 0.5-18% slower on these loops (6144x1024x1024 103.5
-// -> 122 us, 3072^3 499 -> 505, 1024x1024x4096 73.2 -> 74.5); the persistent
-// kernel folds every ring::kFoldRun stages.
+// kernel on their tiles, which must match them bit for bit) sum in MFMA
+// accumulators before each fold into the running sums: 4 stages, 128 k. Eight
+// measured 0.5-18% slower on these loops (6144x1024x1024 103.5 -> 122 us,
+// 3072^3 499 -> 505, 1024x1024x4096 73.2 -> 74.5); the persistent kernel folds
+// every ring::kFoldRun stages.
 constexpr int kFoldStages = 4;
 constexpr int kGroupM = 8;
 

@@ -1,7 +1,7 @@
 """CPU restatement of the fused gate/up/SwiGLU GEMM's addressing
-(gemm_f32_dual_swiglu in jade-compute_amd/csrc/gemm_f32.hip) at the C4 MLP
-shape (x[4096x1024], Wg/Wu [1024x2816]) and at the other shapes the fusion
-rule admits: every global address the kernel reads or writes, every LDS byte
+(gemm_f32_dual_swiglu in jade-compute_amd/csrc/gemm_f32.hip) at 4096x2816
+outputs and at other shapes that the fusion rule admits (those whose products
+run on the persistent kernel alone take that kernel's fused form): every global address the kernel reads or writes, every LDS byte
 its LDS-direct loads write, every LDS float its MFMA operand reads and the
 U hand-off touch, lies inside its buffer, for both of its tiles (128x64, and
 64x64 for the edge columns of a partial last round). The workgroup-to-tile
