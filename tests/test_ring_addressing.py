@@ -1,35 +1,17 @@
-"""CPU restatement of the persistent 128x128 GEMM's addressing
+"""CPU restatement of the persistent 128x128 GEMM's schedule
 (gemm_f32_ring in jade-compute_amd/csrc/gemm_ring.hip): the workgroup-to-tile
-map covers every tile once and gives every workgroup a run of whole tiles;
-each stage's LDS-direct loads fill exactly the A and B regions of their ring
-slot, each 16-byte chunk once, from the tile's A rows and B columns at that
-stage's k; the MFMA operand reads of every quarter read back the values the
-MFMA operand layout needs (A[row][16h + 4q + e], B[16h + 4q + e][2c + j])
-from inside the 128 KiB the kernel declares; the epilogue's stores cover the
-128x128 tile once. The kernel's index formulas are restated with numpy over
-all waves, lanes, loads, quarters and slots."""
+map covers every tile once and gives every workgroup a run of whole tiles; the
+load cursors bring each stage of each tile in turn, past the last one too, from
+inside A and B; no register set is loaded before its stage is converted, none
+converted before it is loaded; the epilogue's stores cover a tile once in every
+form, and the FP32 recomputation reads the rows, columns and k of the outputs
+that it replaces. The LDS side is restated in test_split_addressing.py."""
 import numpy as np
 import pytest
 
 BK, BM, BN = 32, 128, 128
-DEPTH = 4
-A_STAGE_B = BM * BK * 4            # 16 KiB
-B_STAGE_B = BK * BN * 4
-B_REGION = DEPTH * A_STAGE_B       # B slots from 64 KiB
-LDS_BYTES = DEPTH * (A_STAGE_B + B_STAGE_B)
 CUS, GROUP_M = 256, 8
-TM = 1                             # the launched form: eight waves of 32x64
-WAVES, LANES = 8 // TM, 64
-LOADS = 32 // WAVES                # one-KiB loads per wave per stage
-HALF = LOADS // 2
-
-
-def swz_a(row):
-    return (row >> 1) & 7
-
-
-def swz_b(row):
-    return row & 7
+WAVES, LANES = 8, 64
 
 
 def xcd_order(bid, count):
@@ -64,120 +46,100 @@ def test_persistent_map_covers_every_tile_once(tiles_m, tiles_n):
     assert max(runs) - min(runs) <= 1 and sum(runs) == tiles
 
 
-def lane_grid():
-    wave = np.arange(WAVES)[:, None, None]
-    lane = np.arange(LANES)[None, :, None]
-    return wave, lane
+class Cursor:
+    """load_a's or load_b's cursor: (tile, stage) of the next load."""
+
+    def __init__(self, nk):
+        self.nk, self.tile, self.stage = nk, 0, 0
+
+    def take(self, next_tile):
+        at = (self.tile, self.stage)
+        self.stage += 1
+        if self.stage == self.nk:
+            self.tile, self.stage = next_tile, 0
+        return at
 
 
-@pytest.mark.parametrize("n,k", [(4096, 4096), (11008, 4096), (1024, 2816), (128, 256)])
+@pytest.mark.parametrize("n,k", [(4096, 4096), (11008, 4096), (1024, 2816), (128, 512)])
 def test_stage_loads_fill_their_slot_once(n, k):
-    # issue_part: A load x of wave w is instruction w * HALF + x (eight
-    # 128-byte rows of one KiB), B load x instruction w * HALF + x (two
-    # 512-byte rows); lane l writes LDS at M0 + 16 l.
-    wave, lane = lane_grid()
-    x = np.arange(HALF)[None, None, :]
-    inst = wave * HALF + x
-    ra = inst * 8 + (lane >> 3)
-    ja = (lane & 7) ^ swz_a(ra)
-    voa = (ra * k + 4 * ja) * 4                          # bytes from the stage's A base
-    rb = inst * 2 + (lane >> 5)
-    jb = (lane & 31) ^ swz_b(rb)
-    vob = (rb * n + 4 * jb) * 4
-    for slot in range(DEPTH):
-        a_lds = slot * A_STAGE_B + inst * 1024 + lane * 16
-        b_lds = B_REGION + slot * B_STAGE_B + inst * 1024 + lane * 16
-        # Each region filled exactly once, 16 bytes per lane.
-        assert sorted(a_lds.ravel().tolist()) == list(range(slot * A_STAGE_B, (slot + 1) * A_STAGE_B, 16))
-        assert sorted(b_lds.ravel().tolist()) == list(range(B_REGION + slot * B_STAGE_B,
-                                                            B_REGION + (slot + 1) * B_STAGE_B, 16))
-    # Sources: rows [0, 128) x k [0, 32) of A, rows [0, 32) x columns [0, 128)
-    # of B, relative to the stage's bases, each 16-byte chunk once; and the
-    # 32-bit offsets stay below 2^31 (dma_offsets_fit).
-    a_row, a_col = voa // 4 // k, voa // 4 % k
-    assert a_row.min() == 0 and a_row.max() == BM - 1 and a_col.max() <= BK - 4
-    assert len(set(zip(a_row.ravel().tolist(), a_col.ravel().tolist()))) == BM * BK // 4
-    b_row, b_col = vob // 4 // n, vob // 4 % n
-    assert b_row.max() == BK - 1 and b_col.max() <= BN - 4
-    assert len(set(zip(b_row.ravel().tolist(), b_col.ravel().tolist()))) == BK * BN // 4
-    assert voa.max() < 2 ** 31 and vob.max() < 2 ** 31
-    # The physical chunk a lane writes holds logical chunk j ^ swz (A) and
-    # j ^ swz (B) of its row: the layout the operand reads undo.
-    phys_a = (inst * 1024 + lane * 16) % 128 // 16
-    assert np.array_equal(phys_a ^ swz_a(ra), a_col // 4)
-    phys_b = (inst * 1024 + lane * 16) % 512 // 16
-    assert np.array_equal(phys_b ^ swz_b(rb), b_col // 4)
+    # One stage's loads of all threads: rows [0, 128) x k [0, 32) of A and rows
+    # [0, 32) x columns [0, 128) of B (of 64 columns of each product, fused),
+    # each element once, from 32-bit offsets.
+    tid = np.arange(512)
+    wave, lane = tid >> 6, tid & 63
+    a = ((tid >> 2) * k + 8 * (tid & 3))[:, None] + np.arange(8)
+    assert len(set(a.ravel().tolist())) == BM * BK
+    assert (a // k).max() == BM - 1 and (a % k).max() == BK - 1 and 4 * int(a.max()) + 4 < 2 ** 31
+    for cols, width in ((2 * lane, 2), (lane, 1)):
+        b = (4 * wave * n + cols)[:, None, None] + n * np.arange(4)[:, None] + np.arange(width)
+        assert len(set(b.ravel().tolist())) == BK * 64 * width
+        assert (b // n).max() == BK - 1 and (b % n).max() == 64 * width - 1 and 4 * int(b.max()) + 4 < 2 ** 31
 
 
-def test_operand_reads_return_the_mfma_layout():
-    # Fill a model of one slot with (row, k) tags through the load layout,
-    # then restate read_part: A block i of quarter q is the 16 bytes at
-    # aoff[q] + 4096 i + slot * 16K, B row e at boff[q & 1][e] + 4096 (q >> 1)
-    # + slot * 16K. Lane (h, c) of wave (wm, wn) must read A[32 (TM wm + i) +
-    # c][16h + 4q + e] and B[16h + 4q + e][64 wn + 2c + j].
-    lds = np.full(LDS_BYTES // 4, -1, np.int64)
-    slot = 2
-    for row in range(BM):                    # A: logical chunk j of row at j ^ swz_a(row)
-        for kk in range(BK):
-            phys = ((kk // 4) ^ swz_a(row)) * 4 + kk % 4
-            lds[(slot * A_STAGE_B) // 4 + row * BK + phys] = 1_000_000 + row * 1000 + kk
-    for kr in range(BK):                     # B: logical chunk j of row at j ^ swz_b(row)
-        for col in range(BN):
-            phys = ((col // 4) ^ swz_b(kr)) * 4 + col % 4
-            lds[(B_REGION + slot * B_STAGE_B) // 4 + kr * BN + phys] = 2_000_000 + kr * 1000 + col
+@pytest.mark.parametrize("nk,mine", [(16, 1), (16, 3), (88, 2), (24, 5)])
+def test_ring_schedule_never_overwrites_a_live_slot(nk, mine):
+    # Two register sets for A and two for B. Stage g converts B of g + 1, then
+    # loads g + 3 into that set, then converts A of g + 2 and loads g + 4. Every
+    # conversion must find its own stage of its own tile in the set.
+    aim = {"next": min(1, mine - 1)}
+    cursors, sets = {"a": Cursor(nk), "b": Cursor(nk)}, {}
+    done = {"a": [], "b": []}
+
+    def load(matrix, which):
+        assert sets.get((matrix, which)) is None  # the stage before was converted
+        sets[matrix, which] = cursors[matrix].take(aim["next"])
+
+    def convert(matrix, which):
+        done[matrix].append(sets[matrix, which])
+        sets[matrix, which] = None
+
+    for step, matrix, which in ((load, "a", 0), (load, "b", 0), (load, "a", 1), (load, "b", 1), (convert, "a", 0),
+                                (load, "a", 0), (convert, "b", 0), (load, "b", 0), (convert, "a", 1), (load, "a", 1)):
+        step(matrix, which)
+    for tile in range(mine):
+        if tile > 0:
+            aim["next"] = min(tile + 1, mine - 1)
+        for stage in range(nk):
+            p = stage & 1
+            convert("b", p ^ 1)
+            load("b", p ^ 1)
+            convert("a", p)
+            load("a", p)
+    stages = [(tile, stage) for tile in range(mine) for stage in range(nk)]
+    for matrix in ("a", "b"):
+        assert done[matrix][:len(stages)] == stages
+        assert all(tile == mine - 1 for tile, _ in done[matrix][len(stages):])  # read again, never multiplied
+
+
+def outputs(dual):
+    """(wave, lane, accumulator, value) -> (product, row, column) of the tile, as `store` writes them."""
     for wave in range(WAVES):
         wm, wn = wave >> 1, wave & 1
         for lane in range(LANES):
             h, c = lane >> 5, lane & 31
-            aoff = [(wm * 32 * TM + c) * 128 + (((4 * h + q) ^ ((c >> 1) & 7)) << 4) for q in range(4)]
-            boff = [[B_REGION + (16 * h + 4 * p + e) * 512 + (((wn * 16 + (c >> 1)) ^ (4 * p + e)) << 4)
-                     + (c & 1) * 8 for e in range(4)] for p in range(2)]
-            for q in range(4):
-                for i in range(TM):
-                    at = aoff[q] + i * 4096 + slot * A_STAGE_B
-                    assert 0 <= at and at + 16 <= B_REGION
-                    got = lds[at // 4: at // 4 + 4]
-                    row = 32 * (TM * wm + i) + c
-                    assert got.tolist() == [1_000_000 + row * 1000 + 16 * h + 4 * q + e for e in range(4)]
-                for e in range(4):
-                    at = boff[q & 1][e] + (q >> 1) * 4096 + slot * B_STAGE_B
-                    assert B_REGION <= at and at + 8 <= LDS_BYTES
-                    got = lds[at // 4: at // 4 + 2]
-                    kr = 16 * h + 4 * q + e
-                    assert got.tolist() == [2_000_000 + kr * 1000 + 64 * wn + 2 * c + j for j in range(2)]
+            for v in range(16):
+                row = 32 * wm + 4 * h + 8 * (v >> 2) + (v & 3)
+                for j in range(2):
+                    yield (wave, lane, j, v), ((j, row, 32 * wn + c) if dual else (0, row, 64 * wn + 2 * c + j))
 
 
-def test_epilogue_covers_the_tile_once():
-    # store: lane (h, c) of wave (wm, wn) writes rows 32 (TM wm + i) + 8 (v >> 2)
-    # + 4h + (v & 3), columns 64 wn + 2c + j of the tile.
-    seen = {}
-    for wave in range(WAVES):
-        wm, wn = wave >> 1, wave & 1
-        for lane in range(LANES):
-            h, c = lane >> 5, lane & 31
-            for i in range(TM):
-                for v in range(16):
-                    row = 32 * (TM * wm + i) + 8 * (v >> 2) + 4 * h + (v & 3)
-                    for j in range(2):
-                        key = (row, 64 * wn + 2 * c + j)
-                        seen[key] = seen.get(key, 0) + 1
-    assert len(seen) == BM * BN and set(seen.values()) == {1}
+@pytest.mark.parametrize("dual", [False, True])
+def test_epilogue_covers_the_tile_once(dual):
+    seen = [place for _, place in outputs(dual)]
+    assert len(seen) == len(set(seen)) == BM * BN
+    assert max(row for _, row, _ in seen) == BM - 1 and max(col for _, _, col in seen) == (63 if dual else 127)
 
 
-def test_ring_schedule_never_overwrites_a_live_slot():
-    # Model of the issue order: the prologue loads stages 0-2, then iteration
-    # g loads stage g + 3 into slot (g + 3) % 4, LOADS loads per stage. At the
-    # top of iteration g the kernel waits until at most LOADS loads are
-    # outstanding (vmcnt counts loads in issue order), then publishes stage
-    # g + 1 with the barrier; iteration g reads slot g % 4 and, in its last
-    # quarter, stage g + 1's first operands. So stage g + 1 must be complete
-    # at that wait, and the slot loaded during iteration g must be neither of
-    # the two read then. The prologue waits down to 2 LOADS: stage 0.
-    issued = [s for s in range(3) for _ in range(LOADS)]
-    assert set(issued[:len(issued) - 2 * LOADS]) == {0}
-    for g in range(96):
-        complete = issued[:len(issued) - LOADS]       # vmcnt(LOADS)
-        assert complete.count(g + 1) == LOADS and (g + 2) not in complete
-        loading = (g + 3) % DEPTH
-        assert loading not in (g % DEPTH, (g + 1) % DEPTH)
-        issued += [g + 3] * LOADS
+@pytest.mark.parametrize("dual", [False, True])
+def test_operand_reads_return_the_mfma_layout(dual):
+    # The FP32 recomputation: lane (h, c) reads A row 32 wm + c and, for
+    # accumulator j, B column 64 wn + 2c + j (fused: column 32 wn + c of product
+    # j), k 4h + e of every eight. v_mfma_f32_32x32x2_f32 puts row
+    # 8 (v >> 2) + 4h + (v & 3) of A's 32 rows and column c of B's 32 into value v
+    # of lane (h, c): those must be the row and column that `store` writes.
+    assert sorted(4 * h + e for h in range(2) for e in range(4)) == list(range(8))
+    for (wave, lane, j, v), (product, row, col) in outputs(dual):
+        wm, wn, h, c = wave >> 1, wave & 1, lane >> 5, lane & 31
+        a_rows = [32 * wm + i for i in range(32)]
+        b_cols = [(j, 32 * wn + i) if dual else (0, 64 * wn + 2 * i + j) for i in range(32)]
+        assert a_rows[8 * (v >> 2) + 4 * h + (v & 3)] == row and b_cols[c] == (product, col)
