@@ -28,22 +28,13 @@ constexpr uint32_t kRawBuffer = 0x00020000;  // buffer descriptor word 3: raw bu
 constexpr int kSliceK = 32, kCols = 32, kRows = 16, kSlices = 2;
 
 // sum != nullptr: also sum = C + residual (both [M, N]), the stream kernel's
-// FP32 add. Workgroups with blockIdx.y == 1 compute C1 = A1 B1 instead, an
-// independent product of the same shape.
+// FP32 add.
 template <int G>
-__global__ __launch_bounds__(64 * G) void gemm_f32_rows16(const float *__restrict__ A, const float *__restrict__ B,
-                                                          float *__restrict__ C, int M, int N, int K,
-                                                          const float *__restrict__ residual, float *__restrict__ sum,
-                                                          const float *__restrict__ A1, const float *__restrict__ B1,
-                                                          float *__restrict__ C1) {
+__device__ inline void rows16(const float *__restrict__ A, const float *__restrict__ B, float *__restrict__ C, int M,
+                              int N, int K, const float *__restrict__ residual, float *__restrict__ sum) {
     __shared__ float sums[G][kRows][kCols];
     const int lane = int(threadIdx.x) & 63, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
     const int g = lane >> 4, i = lane & 15, n0 = int(blockIdx.x) * kCols;
-    if (blockIdx.y == 1) {
-        A = A1;
-        B = B1;
-        C = C1;
-    }
     // Rows of A past M and rows of B past K lie past the buffers and read
     // zero; a run of A past K reads the next row and is zeroed below.
     const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
@@ -92,36 +83,45 @@ __global__ __launch_bounds__(64 * G) void gemm_f32_rows16(const float *__restric
     }
 }
 
-}  // namespace
+template <int G>
+__global__ __launch_bounds__(64 * G) void gemm_f32_rows16(const float *A, const float *B, float *C, int M, int N,
+                                                          int K, const float *residual, float *sum) {
+    rows16<G>(A, B, C, M, N, K, residual, sum);
+}
 
-namespace {
+// Two independent products of one shape, one in each row of the grid. A kernel
+// of its own: with the choice of pointers in the one above, a launch of one
+// product took 0.05-0.08 us more (1x1000x512 3.09 -> 3.17).
+template <int G>
+__global__ __launch_bounds__(64 * G) void gemm_f32_rows16_pair(const float *A0, const float *B0, float *C0,
+                                                               const float *A1, const float *B1, float *C1, int M,
+                                                               int N, int K) {
+    const bool second = blockIdx.y == 1;
+    rows16<G>(second ? A1 : A0, second ? B1 : B0, second ? C1 : C0, M, N, K, nullptr, nullptr);
+}
 
-hipError_t launch(hipStream_t stream, int waves, unsigned products, const float *a, const float *b, float *c,
-                  uint32_t m, uint32_t n, uint32_t k, const float *residual, float *sum, const float *a1,
-                  const float *b1, float *c1) {
-    if (m > uint32_t(kRows) || k > uint32_t(kSlices * kSliceK * waves)) return hipErrorInvalidValue;
-    const dim3 grid((n + kCols - 1) / kCols, products), block(64 * waves);
-    if (waves == 4)
-        hipLaunchKernelGGL(gemm_f32_rows16<4>, grid, block, 0, stream, a, b, c, int(m), int(n), int(k), residual, sum,
-                           a1, b1, c1);
-    else if (waves == 8)
-        hipLaunchKernelGGL(gemm_f32_rows16<8>, grid, block, 0, stream, a, b, c, int(m), int(n), int(k), residual, sum,
-                           a1, b1, c1);
-    else
-        return hipErrorInvalidValue;
-    return hipGetLastError();
+bool takes(int waves, uint32_t m, uint32_t k) {
+    return (waves == 4 || waves == 8) && m <= uint32_t(kRows) && k <= uint32_t(kSlices * kSliceK * waves);
 }
 
 }  // namespace
 
 hipError_t launch_gemm_rows16(hipStream_t stream, int waves, const float *a, const float *b, float *c, uint32_t m,
                               uint32_t n, uint32_t k, const float *residual, float *sum) {
-    return launch(stream, waves, 1, a, b, c, m, n, k, residual, sum, nullptr, nullptr, nullptr);
+    if (!takes(waves, m, k)) return hipErrorInvalidValue;
+    const dim3 grid((n + kCols - 1) / kCols), block(64 * waves);
+    hipLaunchKernelGGL(waves == 4 ? gemm_f32_rows16<4> : gemm_f32_rows16<8>, grid, block, 0, stream, a, b, c, int(m),
+                       int(n), int(k), residual, sum);
+    return hipGetLastError();
 }
 
 hipError_t launch_gemm_rows16_pair(hipStream_t stream, int waves, const float *a0, const float *b0, float *c0,
                                    const float *a1, const float *b1, float *c1, uint32_t m, uint32_t n, uint32_t k) {
-    return launch(stream, waves, 2, a0, b0, c0, m, n, k, nullptr, nullptr, a1, b1, c1);
+    if (!takes(waves, m, k)) return hipErrorInvalidValue;
+    const dim3 grid((n + kCols - 1) / kCols, 2), block(64 * waves);
+    hipLaunchKernelGGL(waves == 4 ? gemm_f32_rows16_pair<4> : gemm_f32_rows16_pair<8>, grid, block, 0, stream, a0, b0,
+                       c0, a1, b1, c1, int(m), int(n), int(k));
+    return hipGetLastError();
 }
 
 }  // namespace hipk
