@@ -533,8 +533,13 @@ def _find(directory, suffix):
     return found[0] if found else None
 
 
+RING_FORMS = ("Plain", "Pairs", "Dual")  # gemm_ring.hip's RingForm, which a symbol holds as a number
+
+
 def _short(name):
     name = name.replace("jade::hipk::(anonymous namespace)::", "")
+    for value, form in enumerate(RING_FORMS):
+        name = name.replace(f"(RingForm){value}", f"RingForm::{form}")
     name = name[len("void "):] if name.startswith("void ") else name
     return name.split("(")[0] if "(" in name else name
 
@@ -611,7 +616,8 @@ def summarize_rocprof(trace_dir, fetch_dir=None, write_dir=None, bench_log=None)
     what the same counters read for the copy kernel of known size
     (COPY_ELEMENTS). With `bench_log` (the profiled run's output), dispatches
     of the persistent GEMM, whose grid is the same at every shape, are split
-    by shape against the bench's own event-timed medians."""
+    by shape against the bench's own event-timed medians (but for its fused
+    form, which the MLP block alone launches)."""
     trace = _read_csv(_find(trace_dir, "kernel_trace.csv"))
     groups = {}
     for row in trace:
@@ -625,7 +631,7 @@ def summarize_rocprof(trace_dir, fetch_dir=None, write_dir=None, bench_log=None)
     vendor_shapes = vendor_gemm_launches(bench_log) if bench_log else []
     rows = []
     for key, durations in groups.items():
-        if key[0].startswith("gemm_f32_ring") and ring_shapes:
+        if key[0].startswith("gemm_f32_ring") and "Dual" not in key[0] and ring_shapes:
             split = split_by_shape(durations, ring_shapes)
         elif key[0].startswith("Cijk_") and vendor_shapes:
             split = split_by_shape(durations, vendor_shapes)

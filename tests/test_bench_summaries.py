@@ -205,3 +205,9 @@ def test_short_workloads_sample_at_least_a_millisecond(bench, monkeypatch):
 def test_launch_names_their_kernel_and_peak(bench, launch, symbol, parts):
     assert bench.symbol_of(launch) == symbol
     assert bench.peak_of(launch) == (bench.PEAK_PARTS_TFLOPS if parts else bench.PEAK_FP32_MFMA_TFLOPS)
+
+
+def test_ring_forms_are_named(bench):
+    symbol = "void jade::hipk::(anonymous namespace)::gemm_f32_ring<(jade::hipk::(anonymous namespace)::RingForm){}>(float const*)"
+    for value, form in enumerate(("Plain", "Pairs", "Dual")):
+        assert bench._short(symbol.format(value)) == f"gemm_f32_ring<RingForm::{form}>"
