@@ -24,7 +24,8 @@
 // (attention_flash.hip); this kernel takes other head dims, and the split
 // launches, where the parts gain nothing: a slice is a few tiles, and the flash
 // kernel's prologue (two tiles loaded and split before the first product)
-// weighs as much (us, this kernel and that one: H2 S1024 D64 causal 16.0 / 16.9,
+// weighs as much (us, this kernel and that one, whose prologue then waited for
+// its loads one after the other: H2 S1024 D64 causal 16.0 / 16.9,
 // H1 S700 D128 causal 20.7 / 24.8, H2 S513 D32 11.0 / 12.4, H1 S2048 D64 21.9 /
 // 21.4).
 //

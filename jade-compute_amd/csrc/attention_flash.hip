@@ -14,13 +14,19 @@
 // queries and 32 keys), and beside them the VALU: the softmax, splitting the
 // probabilities, and splitting each K and V element once per block. Eight
 // waves share a tile, two per SIMD, so that one wave's softmax runs beside the
-// other's MFMAs. Measured (us) against the FP32-MFMA kernel: H128 S4096 D128
-// causal 4100 -> 2575 (214 TFLOP/s), H64 S2048 D128 noncausal 996 -> 641, H128
-// S4096 D64 causal 2238 -> 1466, H24 S1531 D80 noncausal 411 -> 156 (dims pad
-// to 96 instead of 128, and 144 blocks of 256 queries run in one round where
-// 288 of 128 took two), H32 S1000 D96 noncausal 144 -> 84. Error against FP64
-// (2-norm, relative): 4.1e-7 where that kernel had 5.4e-7 (H128 S4096 D128
-// causal), 6.3e-7 for 7.8e-7 (H24 S1531 D80).
+// other's MFMAs. Measured (us, one box, N(0, 1) operands) against the FP32-MFMA
+// kernel: H128 S4096 D128 causal 4076 -> 2508 (219 TFLOP/s), H64 S2048 D128
+// noncausal 996 -> 610, H128 S4096 D64 causal 2239 -> 1439, H24 S1531 D80
+// noncausal 410 -> 160 (dims pad to 96 instead of 128, and 144 blocks of 256
+// queries run in one round where 288 of 128 took two), H32 S1000 D96 noncausal
+// 149 -> 97. A sequence of one to three key tiles gains least, and a few lose:
+// H512 S64 D128 causal 46.5 -> 23.7, but H304 S31 D128 noncausal 17.1 -> 18.1
+// (one block a CU where that kernel has two), H2 S64 D32 4.8 -> 5.1. Error
+// against FP64 (2-norm, relative): 4.0e-7 where that kernel had 5.4e-7 (H128
+// S4096 D128 causal), 6.3e-7 for 7.8e-7 (H24 S1531 D80).
+//
+// Head dim 128 with four waves and a causal mask fills a SIMD's 512 registers
+// and keeps 17 more in scratch: Q's operands, three of which it reloads a tile.
 //
 // V is scaled before it is split and the outputs are scaled back, Q is scaled
 // up and K down, so every finite V and Q is carried exactly (split_bf16.hpp).

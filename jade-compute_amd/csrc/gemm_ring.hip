@@ -17,8 +17,8 @@ namespace {
 // runs 1.81 PFLOP/s with one wave per SIMD and 1.98 with two, so 300-330
 // TFLOP/s of FP32 products. v_mfma_f32_32x32x2_f32, which this kernel ran on
 // before, tops out at 157 and this kernel reached 150 with it.
-// Measured (us, one box, against that kernel): 4096^3 918 -> 684, 2048^3
-// 120.0 -> 91, 4096x11008x4096 2490 -> 1880. With the staging taken out of a
+// Measured (us, one box, against that kernel): 4096^3 934 -> 691 a call, 2048^3
+// 121 -> 91, 4096x11008x4096 2525 -> 1865 a call. With the staging taken out of a
 // copy (MFMAs and operand reads alone) 4096^3 runs 437 us; global loads, the
 // conversion and the LDS writes each add 60-90 us of issue and waiting that
 // the two waves of a SIMD do not hide. Neither the order of that work (spread
@@ -55,9 +55,11 @@ namespace {
 // sums are not all finite computes its outputs again from global memory with
 // FP32 MFMAs and takes those in the place of the sums that are not, so
 // infinities, NaN and overflow come out as FP32 arithmetic gives them, at about
-// a tenth of the speed. Which way an output is computed thus depends on its own
-// row and column alone, not on its tile's other outputs: every form of this
-// kernel gives it the same bits.
+// a third of the speed (4096^3 with one infinity in B, or with every sum past
+// 2^96, 2200 us; four k steps of loads kept ahead of these products spilled 289
+// registers and ran between 1985 and 2807). Which way an output is computed
+// thus depends on its own row and column alone, not on its tile's other
+// outputs: every form of this kernel gives it the same bits.
 //
 // Requires M, N multiples of 128 (N of 64 for DUAL), K a multiple of 256,
 // 16-byte aligned operands, 32-bit load offsets inside a tile.
