@@ -19,11 +19,11 @@
 // noncausal 996 -> 610, H128 S4096 D64 causal 2239 -> 1439, H24 S1531 D80
 // noncausal 410 -> 160 (dims pad to 96 instead of 128, and 144 blocks of 256
 // queries run in one round where 288 of 128 took two), H32 S1000 D96 noncausal
-// 149 -> 97. A sequence of one to three key tiles gains least, and a few lose:
-// H512 S64 D128 causal 46.5 -> 23.7, but H304 S31 D128 noncausal 17.1 -> 18.1
-// (one block a CU where that kernel has two), H2 S64 D32 4.8 -> 5.1. Error
-// against FP64 (2-norm, relative): 4.0e-7 where that kernel had 5.4e-7 (H128
-// S4096 D128 causal), 6.3e-7 for 7.8e-7 (H24 S1531 D80).
+// 149 -> 97. A sequence of one to three key tiles gains least: H512 S64 D128
+// causal 46.5 -> 21.9, H2 S64 D32 4.8 -> 4.8, and H304 S31 D128 noncausal
+// loses, 17.1 -> 18.0 (one block a CU where that kernel has two). Error against
+// FP64 (2-norm, relative): 4.0e-7 where that kernel had 5.4e-7 (H128 S4096 D128
+// causal), 6.3e-7 for 7.8e-7 (H24 S1531 D80).
 //
 // Head dim 128 with four waves and a causal mask fills a SIMD's 512 registers
 // and keeps 17 more in scratch: Q's operands, three of which it reloads a tile.
@@ -33,8 +33,8 @@
 // What the parts do not carry is noticed and done again from global memory
 // with FP32 MFMAs, per wave: non-finite sums (infinities, NaN or overflow among
 // the operands) and queries past 2^64 in log2 units. With such queries out of
-// the way the bits that a K below 2^-78 loses move no score by more than
-// 2^-38 a dim. Weights below 2^-100 of the reference weight keep fewer than 24 bits.
+// the way the bits that a K below 2^-78 loses move no score by more than 2^-38
+// a dim. Weights below 2^-100 of the reference weight keep fewer than 24 bits.
 #include <type_traits>
 #include <utility>
 
@@ -483,9 +483,12 @@ attention_flash(const float *__restrict__ Q, const float *__restrict__ K, const 
     // Two waves per SIMD: a wave's scores, softmax and P V follow each other and
     // the other wave's matrix work covers its softmax (against the schedule
     // above at H64 S2048 noncausal: D128 641 us for 768, D64 357 for 359). K of tile
-    // t + 1 is converted beside the scores, V beside P V.
-    auto plain_tile = [&](int t, auto wc) __attribute__((always_inline)) {
-        constexpr bool WORK = decltype(wc)::value;
+    // t + 1 is converted beside the scores, V beside P V; the block's last tile
+    // stages nothing (without STAGE H2 S64 D32 takes 5.1 us for 4.8, H256 S64
+    // D32 6.0 for 5.6, H256 S300 D72 55.8 for 52.1; the schedule above spills
+    // with such a form).
+    auto plain_tile = [&](int t, auto wc, auto gc) __attribute__((always_inline)) {
+        constexpr bool WORK = decltype(wc)::value, STAGE = decltype(gc)::value;
         const uint32_t cur = uint32_t(t) & 1u, other = cur ^ 1u;
         f32x16 sn[2] = {};
         if constexpr (WORK) {
@@ -505,7 +508,7 @@ attention_flash(const float *__restrict__ Q, const float *__restrict__ K, const 
                 if constexpr (s + 1 < KS && p == 1) read_q(s + 1);
             }
             constexpr int lo = kFirstEvent<n, 12, kSlots1>, hi = kFirstEvent<n + 1, 12, kSlots1>;
-            each<hi - lo>([&](auto ec) __attribute__((always_inline)) {
+            each<STAGE ? hi - lo : 0>([&](auto ec) __attribute__((always_inline)) {
                 constexpr int x = lo + decltype(ec)::value;
                 convert_k(0, x / 3, x % 3);
                 if constexpr (x % 6 == 5) load_k(0, x / 6, t + 2);
@@ -584,7 +587,7 @@ attention_flash(const float *__restrict__ Q, const float *__restrict__ K, const 
                 }
             }
             constexpr int lo = kFirstEvent<n, 6 * kPairsV, kSlots2 - 4>, hi = kFirstEvent<n + 1, 6 * kPairsV, kSlots2 - 4>;
-            each<hi - lo>([&](auto ec) __attribute__((always_inline)) {
+            each<STAGE ? hi - lo : 0>([&](auto ec) __attribute__((always_inline)) {
                 constexpr int e = lo + decltype(ec)::value, v = e / (3 * kPairsV), u = e / 3 % kPairsV, x = e % 3;
                 convert_v(v, u, x);
                 if constexpr (x == 2) {
@@ -599,15 +602,16 @@ attention_flash(const float *__restrict__ Q, const float *__restrict__ K, const 
             });
             if constexpr (WORK) __builtin_amdgcn_sched_barrier(0);
         });
-        publish();
+        if constexpr (STAGE) publish();
     };
     if constexpr (S::kPlain) {
-        for (int t = 0; t < t_end; ++t) {
+        for (int t = 0; t < t_end - 1; ++t) {
             if (live(t))
-                plain_tile(t, std::true_type{});
+                plain_tile(t, std::true_type{}, std::true_type{});
             else
-                plain_tile(t, std::false_type{});
+                plain_tile(t, std::false_type{}, std::true_type{});
         }
+        if (live(t_end - 1)) plain_tile(t_end - 1, std::true_type{}, std::false_type{});
     } else {
         for (int t = 0; t < t_end; ++t) {
             if (live(t + 1))
